@@ -204,7 +204,8 @@ struct WfSpectral {
 enum { WF_F_ITER = 0, WF_F_FIRST = 1, WF_F_CONST = 2, WF_F_TOP = 3 };
 
 hipError_t wf_launch_pressure_rhs_fx(const WfConst &c, const WfSpectral &sp, const WfState &Ys, const WfState &Yn,
-                                     const wf_real *p, int mode, hipStream_t s);
+                                     const wf_real *p, int mode, double tol, double rtol, int check, int max_iter,
+                                     hipStream_t s);
 hipError_t wf_launch_fy(const WfSpectral &sp, wf_real2 *buf, long slab_stride, int slab0, int nslabs, int sign,
                         int guarded, hipStream_t s);
 hipError_t wf_launch_density(const WfConst &c, const wf_real *T, wf_real *rho, hipStream_t s);
@@ -229,7 +230,7 @@ struct WfPressItem {
 };
 hipError_t wf_launch_density_batch(const WfConst &c, const WfPressItem *tab, int nm, hipStream_t s);
 hipError_t wf_launch_iter_reset_batch(const WfPressItem *tab, int nm, hipStream_t s);
-hipError_t wf_launch_pressure_rhs_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, int mode,
+hipError_t wf_launch_pressure_rhs_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, int mode, int check,
                                            hipStream_t s);
 hipError_t wf_launch_fy_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, long slab_stride, int slab0,
                               int nslabs, int sign, int guarded, hipStream_t s);

@@ -219,9 +219,16 @@ __device__ __forceinline__ void wf_reduce_max(const double *a, int n, double *ou
  * also stops once err <= rtol max|p_new|: below that the FP32 iteration no
  * longer moves p toward the solution (its accuracy floor).  The flag and the
  * solve count are also written to mapped host memory so the host can stop
- * queueing solves without a round trip.  (A separate one-workgroup launch: on
- * a multi-XCD device a grid-wide reduction inside the inverse transform would
- * need a device-scope release, an L2 write-back, in every workgroup.) */
+ * queueing solves without a round trip.
+ *
+ * The check of solve m is done by one extra workgroup (block 0) of solve
+ * m + 1's first pass, beside the pass's own workgroups; only the last queued
+ * solve is checked by a launch of its own (k_iter_check).  If m converged,
+ * that first pass has written F, which nothing reads any more, and every
+ * later pass returns at once.  As its own launch after every solve the check
+ * took 4.3-6.2 us of latency, 5 % of a solve at 256x256x128 and 12-17 % at
+ * 64x64x32 and below.  (Reducing in the inverse transform itself would need a
+ * device-scope release, an L2 write-back, in every workgroup.) */
 __device__ __forceinline__ void wf_iter_check_body(const WfSpectral &sp, double tol, double rtol, int m,
                                                    int max_iter) {
     WfIterCtl *ctl = sp.ctl;
@@ -256,6 +263,15 @@ __global__ __launch_bounds__(WF_NT) void k_iter_check(WfSpectral sp, double tol,
     wf_iter_check_body(sp, tol, rtol, m, max_iter);
 }
 
+/* Block index of a first pass whose block 0 checks the previous solve
+ * (check >= 0: its index), -1 for that block after the check. */
+__device__ __forceinline__ int wf_checked_block(const WfSpectral &sp, double tol, double rtol, int check,
+                                                int max_iter) {
+    if (check < 0) return (int)blockIdx.x;
+    if (blockIdx.x == 0) wf_iter_check_body(sp, tol, rtol, check, max_iter);
+    return (int)blockIdx.x - 1;
+}
+
 /* Input value of the x-transform at (i, j, k) for form MODE. */
 template <int MODE>
 __device__ __forceinline__ wf_real wf_fx_input(const WfConst &c, const WfSpectral &sp, const WfState &Ys,
@@ -279,7 +295,7 @@ __device__ __forceinline__ wf_real wf_fx_input(const WfConst &c, const WfSpectra
  * half-spectrum into F[k][kx][j].  NX > 0 selects the compile-time plan. */
 template <int NX, int MODE>
 __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectral &sp, const WfState &Ys,
-                                               const WfState &Yn, const wf_real *p) {
+                                               const WfState &Yn, const wf_real *p, int block, int nblocks) {
     if (MODE != WF_F_TOP && sp.ctl->done) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
@@ -289,7 +305,7 @@ __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectra
     const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
     wfc *tw = smem, *bufa = smem + nx, *bufb = bufa + pairs * nx;
     int g, ks;
-    wf_tile_decode(sp.ngroups, (MODE == WF_F_TOP) ? 1 : sp.nz - 1, &g, &ks);
+    wf_tile_decode_at(block, nblocks, sp.ngroups, (MODE == WF_F_TOP) ? 1 : sp.nz - 1, &g, &ks);
     const int k = (MODE == WF_F_TOP) ? c.Nz - 1 : 1 + ks;
     const int j0 = 2 * g * pairs;
     for (int t = threadIdx.x; t < nx; t += blockDim.x) tw[t] = *(const wfc *)&sp.twx[t];
@@ -357,8 +373,10 @@ __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectra
 }
 template <int NX, int MODE>
 __global__ __launch_bounds__(WF_NT) void k_rhs_fx(WfConst c, WfSpectral sp, WfState Ys, WfState Yn,
-                                                  const wf_real *p) {
-    wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p);
+                                                  const wf_real *p, double tol, double rtol, int check,
+                                                  int max_iter) {
+    const int b = wf_checked_block(sp, tol, rtol, check, max_iter);
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p, b, (int)gridDim.x - (check >= 0));
 }
 
 /* P2/P4: y-transform of sp.fy_cols kx columns (each contiguous over ky) of
@@ -1118,9 +1136,10 @@ __global__ void k_iter_reset_batch(const WfPressItem *__restrict__ tab) {
 }
 
 template <int NX, int MODE>
-__global__ __launch_bounds__(WF_NT) void k_rhs_fx_batch(const WfPressItem *__restrict__ tab) {
+__global__ __launch_bounds__(WF_NT) void k_rhs_fx_batch(const WfPressItem *__restrict__ tab, int check) {
     const WfPressItem it = wf_press_load(tab);
-    wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p);
+    const int b = wf_checked_block(it.sp, it.tol, it.rtol, check, it.max_iter);
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, (int)gridDim.x - (check >= 0));
 }
 
 /* twy: the class's y twiddle table (it depends on ny alone, so every member's
@@ -1223,15 +1242,24 @@ hipError_t wf_launch_iter_reset(WfIterCtl *ctl, hipStream_t s) {
 }
 
 hipError_t wf_launch_pressure_rhs_fx(const WfConst &c, const WfSpectral &sp, const WfState &Ys, const WfState &Yn,
-                                     const wf_real *p, int mode, hipStream_t s) {
+                                     const wf_real *p, int mode, double tol, double rtol, int check, int max_iter,
+                                     hipStream_t s) {
     const int nslabs = (mode == WF_F_TOP) ? 1 : sp.nz - 1;
-    dim3 grd((unsigned)(sp.ngroups * nslabs));
+    dim3 grd((unsigned)(sp.ngroups * nslabs + (check >= 0)));
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
     switch (mode) {
-        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p); break;
-        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p); break;
-        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p); break;
-        default: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_TOP, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p); break;
+        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
+                                        check, max_iter);
+            break;
+        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
+                                        check, max_iter);
+            break;
+        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
+                                        check, max_iter);
+            break;
+        default: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_TOP, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
+                                        check, max_iter);
+            break;
     }
     return hipGetLastError();
 }
@@ -1300,15 +1328,15 @@ hipError_t wf_launch_iter_reset_batch(const WfPressItem *tab, int nm, hipStream_
     return hipGetLastError();
 }
 
-hipError_t wf_launch_pressure_rhs_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, int mode,
+hipError_t wf_launch_pressure_rhs_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, int mode, int check,
                                            hipStream_t s) {
     const int nslabs = (mode == WF_F_TOP) ? 1 : sp.nz - 1;
-    dim3 grd((unsigned)(sp.ngroups * nslabs), 1, nm);
+    dim3 grd((unsigned)(sp.ngroups * nslabs + (check >= 0)), 1, nm);
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
     switch (mode) {
-        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, tab); break;
-        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, tab); break;
-        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, tab); break;
+        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, tab, check); break;
+        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, tab, check); break;
+        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, tab, check); break;
         default: return hipErrorInvalidValue; /* the top plane is solo only */
     }
     return hipGetLastError();

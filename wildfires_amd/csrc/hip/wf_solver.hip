@@ -636,7 +636,7 @@ static int wf_get_field(Solver *s, const wf_real *src, double *f_host) {
  * writes the unique nodes of k = Nz-1) */
 static int wf_top_spectrum(Solver *s) {
     WfState none = {nullptr, nullptr, nullptr, nullptr, nullptr};
-    WF_HIP(wf_launch_pressure_rhs_fx(s->c, s->sp, none, none, s->p, WF_F_TOP, s->stream));
+    WF_HIP(wf_launch_pressure_rhs_fx(s->c, s->sp, none, none, s->p, WF_F_TOP, 0.0, 0.0, -1, 0, s->stream));
     WF_HIP(wf_launch_fy(s->sp, s->Ptop, 0, 0, 1, -1, 0, s->stream));
     return WF_OK;
 }
@@ -760,17 +760,24 @@ static int wf_pressure_begin(Solver *s, const WfState &yn) {
     return WF_OK;
 }
 
-/* solve m of the iteration and its convergence check (launches only) */
-static int wf_pressure_one(Solver *s, const WfState &ys, const WfState &yn, int m, int max_iter) {
+/* solve m of the iteration (launches only).  Its first pass checks the
+ * convergence of solve m - 1 when check is set; the last solve queued (last)
+ * is checked by a launch of its own. */
+static int wf_pressure_one(Solver *s, const WfState &ys, const WfState &yn, int m, int max_iter, bool check,
+                           bool last) {
     const Parameters &P = s->P;
     const long sstride = (long)s->sp.hx * s->sp.ldj;
     const int form = (m > 0) ? WF_F_ITER : (P.variable_density ? WF_F_FIRST : WF_F_CONST);
-    WF_LAUNCH(s, WF_K_PRHS, wf_launch_pressure_rhs_fx(s->c, s->sp, ys, yn, s->p, form, s->stream));
+    WF_LAUNCH(s, WF_K_PRHS,
+              wf_launch_pressure_rhs_fx(s->c, s->sp, ys, yn, s->p, form, P.pressure_solver_tol, s->press_rtol,
+                                        check ? m - 1 : -1, max_iter, s->stream));
     WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 1, s->sp.nz - 1, -1, 1, s->stream));
     WF_LAUNCH(s, WF_K_THOMAS, wf_launch_thomas(s->sp, s->stream));
     WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 0, s->sp.nz, +1, 1, s->stream));
     WF_LAUNCH(s, WF_K_PINV, wf_launch_inverse_fx(s->c, s->sp, s->p, s->stream));
-    WF_LAUNCH(s, WF_K_OTHER, wf_launch_iter_check(s->sp, P.pressure_solver_tol, s->press_rtol, m, max_iter, s->stream));
+    if (last)
+        WF_LAUNCH(s, WF_K_OTHER,
+                  wf_launch_iter_check(s->sp, P.pressure_solver_tol, s->press_rtol, m, max_iter, s->stream));
     return WF_OK;
 }
 
@@ -787,10 +794,13 @@ static int wf_pressure_rest(Solver *s, const WfState &ys, const WfState &yn, int
     int rc;
     for (int m = m0; m < max_iter; m++) {
         if (m > 0 && hf[0]) break;
-        if ((rc = wf_pressure_one(s, ys, yn, m, max_iter))) return rc;
+        /* the solves before m0 have been checked */
+        if ((rc = wf_pressure_one(s, ys, yn, m, max_iter, m > m0, m + 1 >= max_iter))) return rc;
         if (m + 1 >= max_iter) break;
-        /* wait until the device is within WF_LOOKAHEAD solves; if the stream
-         * drains without the flag advancing, fall through and keep queueing */
+        /* wait until the device is within WF_LOOKAHEAD solves (the count
+         * lags a solve: solve m is counted by solve m + 1's first pass); if
+         * the stream drains without the flag advancing, fall through and keep
+         * queueing */
         while (!hf[0] && (m + 1) - hf[1] >= WF_LOOKAHEAD) {
             if (hipStreamQuery(s->stream) == hipSuccess) break;
         }
@@ -1420,12 +1430,12 @@ static int ens_pressure_class(Ensemble *e, int par, int q, hipStream_t st) {
     const long sstride = (long)sp.hx * sp.ldj;
     for (int m = 0; m < e->budget && m < max_iter; m++) {
         const int form = (m > 0) ? WF_F_ITER : (s0->P.variable_density ? WF_F_FIRST : WF_F_CONST);
-        WF_HIP(wf_launch_pressure_rhs_fx_batch(sp, tab, nm, form, st));
+        WF_HIP(wf_launch_pressure_rhs_fx_batch(sp, tab, nm, form, m - 1, st));
         WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 1, sp.nz - 1, -1, 1, st));
         WF_HIP(wf_launch_thomas_batch(sp, tab, nm, st));
         WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 0, sp.nz, +1, 1, st));
         WF_HIP(wf_launch_inverse_fx_batch(sp, tab, nm, st));
-        WF_HIP(wf_launch_iter_check_batch(tab, nm, m, st));
+        if (m + 1 >= e->budget || m + 1 >= max_iter) WF_HIP(wf_launch_iter_check_batch(tab, nm, m, st));
     }
     return WF_OK;
 }
@@ -1454,7 +1464,8 @@ static int ens_enqueue(Ensemble *e, int par) {
             if ((rc = wf_pressure_begin(s, yn))) break;
             const int max_iter = wf_max_iter(s->P);
             for (int m = 0; m < e->budget && m < max_iter; m++)
-                if ((rc = wf_pressure_one(s, ys, yn, m, max_iter))) break;
+                if ((rc = wf_pressure_one(s, ys, yn, m, max_iter, m > 0, m + 1 >= e->budget || m + 1 >= max_iter)))
+                    break;
         }
     }
     for (int i = 0; i < e->n; i++) e->m[i]->stream = e->stream;
