@@ -19,6 +19,8 @@ HOST_SOURCES = ["params.c", "terrain.c", "init.c", "output.c", "solver.c"]
 # compiled once per precision: WF_MIXED=0 (namespace wf64, FP64) and WF_MIXED=1
 # (namespace wf32, the mixed form; any implicit FP32 -> FP64 promotion is an error)
 HIP_PRECISION_SOURCES = ["wf_stage.hip", "wf_pressure.hip", "wf_project.hip", "wf_reports.hip", "wf_solver.hip"]
+# compiled for FP64 alone (namespace wf64)
+HIP_FP64_SOURCES = ["wf_planes.hip"]
 # compiled once: the C-ABI over both precisions, the closure trainer and the
 # static scratch of the entry points that allocate nothing
 HIP_SOURCES = ["wf_api.hip", "wf_closure_train.hip", "wf_noalloc.hip"]
@@ -60,6 +62,10 @@ def build(verbose=False, jobs=None):
             obj = os.path.join(OUT, src + "." + tag + ".o")
             cmds.append([_hipcc()] + HIPCC_FLAGS + flags + ["-c", os.path.join(CSRC, "hip", src), "-o", obj])
             objs.append(obj)
+    for src in HIP_FP64_SOURCES:
+        obj = os.path.join(OUT, src + ".64.o")
+        cmds.append([_hipcc()] + HIPCC_FLAGS + ["-DWF_MIXED=0", "-c", os.path.join(CSRC, "hip", src), "-o", obj])
+        objs.append(obj)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB + ".tmp"] + objs + ["-lm", "-lpthread"],

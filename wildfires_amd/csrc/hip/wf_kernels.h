@@ -5,6 +5,8 @@
 #ifndef WF_KERNELS_H
 #define WF_KERNELS_H
 
+#include <vector>
+
 #include "wf_common.h"
 #include "wf_closure.h"
 
@@ -180,7 +182,7 @@ struct WfSpectral {
     const wf_real *kx2;  /* hx: kx^2 of the retained x-wavenumbers */
     const wf_real *ky2;  /* ny */
     const wf_real *ta;   /* nz-1: sub-diagonal a_k (k-only) */
-    const wf_real *tc;   /* nz-1: super-diagonal c_k for k >= 1 (c_0 depends on K^2) */
+    const wf_real *tc;   /* nz-1: super-diagonal c_k for k >= 1 (c_0 depends on K^2), 0 up to a multiple of 16 */
     /* the same tables in FP64, for the systems solved in FP64 (all of them in
      * the wf64 compilation, the lowest wavenumbers in the mixed one) */
     const double *kx2d, *ky2d, *tad, *tcd, *betad;
@@ -196,6 +198,14 @@ struct WfSpectral {
     const wf_real *rho;            /* rho^n on every node (variable density) */
     WfIterCtl *ctl;
     int *hflag;                    /* mapped host memory: [0] done, [1] solves finished */
+    /* coefficient-plane form (wf_planes.hip, FP64), used when pl is set */
+    int pl;
+    int pl_ld;          /* row stride of a plane: ny rounded up to 16 */
+    int pl_groups;      /* 16-row groups per slab */
+    int pl_nt;          /* threads of the plane solve; 0: its planes do not fit LDS */
+    wf_real *U;         /* [nx][nz][pl_ld] planes of real x-coefficients */
+    const wf_real *pl_fx, *pl_ix, *pl_fy, *pl_iy; /* MFMA operands of the transforms (wf_pl_matrix) */
+    wf_real *pl_l, *pl_ru;  /* [hx][nz up to 16][ny/2+1]: Thomas multipliers l_k and reciprocal pivots 1/u_k */
 };
 
 /* Forms of the x-transform input: the Poisson RHS of a later iteration (stored
@@ -214,6 +224,20 @@ hipError_t wf_launch_thomas(const WfSpectral &sp, hipStream_t s);
 hipError_t wf_launch_pivots(const WfSpectral &sp, double *UB, hipStream_t s);
 hipError_t wf_launch_inverse_fx(const WfConst &c, const WfSpectral &sp, wf_real *p, hipStream_t s);
 hipError_t wf_launch_iter_check(const WfSpectral &sp, double tol, double rtol, int m, int max_iter, hipStream_t s);
+
+/* Coefficient-plane form of the solve (wf_planes.hip). */
+#define WF_PL_ROWS 16     /* rows per workgroup in the x-transforms */
+#define WF_PL_LEN_MAX 512 /* longest transform */
+/* whether the form takes an nx x ny x nz solve, and the threads of its plane solve */
+bool wf_pl_takes(int nx, int ny, int nz, int *nt);
+/* MFMA operand tables of a real transform of length n: forward and inverse */
+void wf_pl_matrix(int n, std::vector<double> &fwd, std::vector<double> &inv);
+hipError_t wf_pl_prepare(const WfSpectral &sp, hipStream_t s);
+hipError_t wf_launch_pl_rhs(const WfConst &c, const WfSpectral &sp, const WfState &Ys, const WfState &Yn,
+                            const wf_real *p, int mode, double tol, double rtol, int check, int max_iter,
+                            hipStream_t s);
+hipError_t wf_launch_pl_solve(const WfSpectral &sp, hipStream_t s);
+hipError_t wf_launch_pl_inv(const WfConst &c, const WfSpectral &sp, wf_real *p, hipStream_t s);
 
 /* One member's operands for the batched pressure passes of an ensemble.  The
  * members of a size class (same grid, precision and iteration limit) run each
@@ -237,6 +261,10 @@ hipError_t wf_launch_fy_batch(const WfSpectral &sp, const WfPressItem *tab, int 
 hipError_t wf_launch_thomas_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s);
 hipError_t wf_launch_inverse_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s);
 hipError_t wf_launch_iter_check_batch(const WfPressItem *tab, int nm, int m, hipStream_t s);
+hipError_t wf_launch_pl_rhs_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, int mode, int check,
+                                  hipStream_t s);
+hipError_t wf_launch_pl_solve_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s);
+hipError_t wf_launch_pl_inv_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s);
 
 /* Temperature source applied at the end of a step (src/cu/functions.cu:325-403). */
 struct WfSource {

@@ -71,6 +71,7 @@ struct Solver {
     unsigned clq_cap;
     int clq_parity; /* which of the two counter sets the next derived pass appends to */
     int *cut, *nzy, *radx, *rady;
+    wf_real *U, *pl_tab, *pl_piv; /* coefficient-plane form of the pressure solve */
     wf_real2 *twx, *twy;
     double *scratch; /* S doubles: host transfers in the reference layout */
     wf_real *Tsrc, *rho;
@@ -434,6 +435,12 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     sp.fy_cols = wf_f2_n1(sp.ny) ? wf_f2_nseq(sp.ny) : WF_FY_COLS;
     sp.ngroups = ((sp.ny + 1) / 2 + sp.fx_pairs - 1) / sp.fx_pairs;
     sp.npmax = sp.ngroups * sp.nz + 1;
+#if !WF_MIXED
+    sp.pl = wf_pl_takes(sp.nx, sp.ny, sp.nz, &sp.pl_nt) ? 1 : 0;
+#endif
+    sp.pl_ld = (sp.ny + 15) & ~15;
+    sp.pl_groups = (sp.ny + WF_PL_ROWS - 1) / WF_PL_ROWS;
+    if (sp.pl) sp.npmax = sp.pl_groups * sp.nz + 1;
     int radx[WF_MAX_RADICES], rady[WF_MAX_RADICES];
     if (wf_factor(sp.nx, radx) < 0 || wf_factor(sp.ny, rady) < 0)
         return wf_fail(WF_E_ARG, "transform length has too many factors");
@@ -455,7 +462,7 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     for (int q = 0; q < sp.ny; q++) ky2[q] = P->ky[q] * P->ky[q];
     if ((rc = wf_upload_real(&s->kx2, kx2.data(), sp.hx))) return rc;
     if ((rc = wf_upload_real(&s->ky2, ky2.data(), sp.ny))) return rc;
-    std::vector<double> ta(sp.nz, 0.0), tc(sp.nz, 0.0), beta(sp.nz, 0.0);
+    std::vector<double> ta(sp.nz, 0.0), tc((sp.nz + 15) & ~15, 0.0), beta(sp.nz, 0.0);
     for (int k = 0; k < Nz - 2; k++) {
         double dz_k = z[k + 1] - z[k], dz_kp1 = z[k + 2] - z[k + 1];
         ta[k] = 2 / (dz_k * (dz_k + dz_kp1));
@@ -466,13 +473,13 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
         }
     }
     if ((rc = wf_upload_real(&s->ta, ta.data(), sp.nz))) return rc;
-    if ((rc = wf_upload_real(&s->tc, tc.data(), sp.nz))) return rc;
+    if ((rc = wf_upload_real(&s->tc, tc.data(), tc.size()))) return rc;
     if ((rc = wf_upload_real(&s->beta, beta.data(), sp.nz))) return rc;
 #if WF_MIXED
     if ((rc = wf_upload(&s->kx2d, kx2.data(), sp.hx))) return rc;
     if ((rc = wf_upload(&s->ky2d, ky2.data(), sp.ny))) return rc;
     if ((rc = wf_upload(&s->tad, ta.data(), sp.nz))) return rc;
-    if ((rc = wf_upload(&s->tcd, tc.data(), sp.nz))) return rc;
+    if ((rc = wf_upload(&s->tcd, tc.data(), tc.size()))) return rc;
     if ((rc = wf_upload(&s->betad, beta.data(), sp.nz))) return rc;
     /* the systems solved in FP64: kx index < low_kx and ky index within
      * low_ky of 0 or ny (WF_MIXED_LOW_KX / WF_MIXED_LOW_KY override 4, 4) */
@@ -491,18 +498,44 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     sp.b0 = -1.0 / dz0;
     sp.beta_top = 2 / (dzNm2 * dzNm1);
     sp.top_div = 2 / (dzNm1 * (dzNm2 + dzNm1));
-    long nspec = (long)sp.nz * sp.hx * sp.ldj;
-    WF_HIP(hipMalloc((void **)&s->F, sizeof(wf_real2) * nspec));
-    WF_HIP(hipMemset(s->F, 0, sizeof(wf_real2) * nspec));
-    WF_HIP(hipMalloc((void **)&s->Ptop, sizeof(wf_real2) * (long)sp.hx * sp.ldj));
-    WF_HIP(hipMemset(s->Ptop, 0, sizeof(wf_real2) * (long)sp.hx * sp.ldj));
     /* 4 levels per half-wave chunk (k_thomas_h) up to 128 levels, else whole-wave chunks of 8 or 16 */
     sp.thomas_lc = (WF_THOMAS_HALF && sp.nz <= 4 * 2 * WF_THOMAS_MAX_CHUNKS) ? 4
                    : (sp.nz <= 8 * WF_THOMAS_MAX_CHUNKS)                       ? 8
                                                                                : 16;
-    const int nchunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
-    WF_HIP(hipMalloc((void **)&s->UB, sizeof(double) * (long)nchunks * sp.hx * sp.ldj));
-    WF_HIP(hipMemset(s->UB, 0, sizeof(double) * (long)nchunks * sp.hx * sp.ldj));
+    if (sp.pl) {
+        const int len[2] = {sp.nx, sp.ny};
+        std::vector<double> tab;
+        size_t at[5] = {0, 0, 0, 0, 0};
+#if !WF_MIXED
+        for (int q = 0; q < 4; q++) { /* forward and inverse tables in x, then in y */
+            std::vector<double> fwd, inv;
+            wf_pl_matrix(len[q / 2], fwd, inv);
+            const std::vector<double> &t = (q & 1) ? inv : fwd;
+            tab.insert(tab.end(), t.begin(), t.end());
+            at[q + 1] = tab.size();
+        }
+#endif
+        if ((rc = wf_upload_real(&s->pl_tab, tab.data(), tab.size()))) return rc;
+        sp.pl_fx = s->pl_tab + at[0];
+        sp.pl_ix = s->pl_tab + at[1];
+        sp.pl_fy = s->pl_tab + at[2];
+        sp.pl_iy = s->pl_tab + at[3];
+        WF_HIP(hipMalloc((void **)&s->U, sizeof(wf_real) * (size_t)sp.nx * sp.nz * sp.pl_ld));
+        const size_t piv = (size_t)sp.hx * ((sp.nz + 15) & ~15) * (sp.ny / 2 + 1);
+        WF_HIP(hipMalloc((void **)&s->pl_piv, sizeof(wf_real) * 2 * piv));
+        sp.U = s->U;
+        sp.pl_l = s->pl_piv;
+        sp.pl_ru = s->pl_piv + piv;
+    } else {
+        const long nspec = (long)sp.nz * sp.hx * sp.ldj;
+        const int nchunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
+        WF_HIP(hipMalloc((void **)&s->F, sizeof(wf_real2) * nspec));
+        WF_HIP(hipMemset(s->F, 0, sizeof(wf_real2) * nspec));
+        WF_HIP(hipMalloc((void **)&s->Ptop, sizeof(wf_real2) * (long)sp.hx * sp.ldj));
+        WF_HIP(hipMemset(s->Ptop, 0, sizeof(wf_real2) * (long)sp.hx * sp.ldj));
+        WF_HIP(hipMalloc((void **)&s->UB, sizeof(double) * (long)nchunks * sp.hx * sp.ldj));
+        WF_HIP(hipMemset(s->UB, 0, sizeof(double) * (long)nchunks * sp.hx * sp.ldj));
+    }
     WF_HIP(hipMalloc((void **)&s->pmax, sizeof(double) * 2 * sp.npmax));
     WF_HIP(hipMemset(s->pmax, 0, sizeof(double) * 2 * sp.npmax));
 #if WF_MIXED
@@ -543,7 +576,10 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     sp.rho = s->rho;
     sp.ctl = s->ctl;
     sp.hflag = s->hflag_dev;
-    WF_HIP(wf_launch_pivots(sp, s->UB, s->stream));
+#if !WF_MIXED
+    if (sp.pl) WF_HIP(wf_pl_prepare(sp, s->stream));
+#endif
+    if (!sp.pl) WF_HIP(wf_launch_pivots(sp, s->UB, s->stream));
     WF_HIP(hipStreamSynchronize(s->stream));
     for (int q = 0; q < 2 * WF_MAX_EVENTS; q++) WF_HIP(hipEventCreate(&s->ev[q]));
     return WF_OK;
@@ -574,7 +610,7 @@ int destroy(Solver *s) {
                     s->cl_prm, s->cl_frag, s->clq_count, s->clq_node, s->clq_x, s->clq_rho, s->topo, s->kx2, s->ky2, s->ta,
                     s->tc, s->beta, s->x, s->y, s->cut, s->nzy, s->radx, s->rady, s->twx, s->twy, s->scratch,
                     s->Tsrc, s->rho, s->ctl, s->kx2d, s->ky2d, s->tad, s->tcd, s->betad,
-                    s->in_box, s->rep_part, s->rep_nan};
+                    s->in_box, s->rep_part, s->rep_nan, s->U, s->pl_tab, s->pl_piv};
     for (size_t q = 0; q < sizeof(bufs) / sizeof(bufs[0]); q++)
         if (bufs[q]) (void)hipFree(bufs[q]);
     for (int q = 0; q < 2 * WF_MAX_EVENTS; q++)
@@ -635,6 +671,7 @@ static int wf_get_field(Solver *s, const wf_real *src, double *f_host) {
 /* spectrum of the top pressure plane (fixed for the whole run: the solve never
  * writes the unique nodes of k = Nz-1) */
 static int wf_top_spectrum(Solver *s) {
+    if (s->sp.pl) return WF_OK; /* its right-hand side reads the plane itself */
     WfState none = {nullptr, nullptr, nullptr, nullptr, nullptr};
     WF_HIP(wf_launch_pressure_rhs_fx(s->c, s->sp, none, none, s->p, WF_F_TOP, 0.0, 0.0, -1, 0, s->stream));
     WF_HIP(wf_launch_fy(s->sp, s->Ptop, 0, 0, 1, -1, 0, s->stream));
@@ -768,13 +805,25 @@ static int wf_pressure_one(Solver *s, const WfState &ys, const WfState &yn, int 
     const Parameters &P = s->P;
     const long sstride = (long)s->sp.hx * s->sp.ldj;
     const int form = (m > 0) ? WF_F_ITER : (P.variable_density ? WF_F_FIRST : WF_F_CONST);
-    WF_LAUNCH(s, WF_K_PRHS,
-              wf_launch_pressure_rhs_fx(s->c, s->sp, ys, yn, s->p, form, P.pressure_solver_tol, s->press_rtol,
-                                        check ? m - 1 : -1, max_iter, s->stream));
-    WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 1, s->sp.nz - 1, -1, 1, s->stream));
-    WF_LAUNCH(s, WF_K_THOMAS, wf_launch_thomas(s->sp, s->stream));
-    WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 0, s->sp.nz, +1, 1, s->stream));
-    WF_LAUNCH(s, WF_K_PINV, wf_launch_inverse_fx(s->c, s->sp, s->p, s->stream));
+    const int chk = check ? m - 1 : -1;
+#if !WF_MIXED
+    if (s->sp.pl) {
+        WF_LAUNCH(s, WF_K_PRHS,
+                  wf_launch_pl_rhs(s->c, s->sp, ys, yn, s->p, form, P.pressure_solver_tol, s->press_rtol, chk,
+                                   max_iter, s->stream));
+        WF_LAUNCH(s, WF_K_THOMAS, wf_launch_pl_solve(s->sp, s->stream));
+        WF_LAUNCH(s, WF_K_PINV, wf_launch_pl_inv(s->c, s->sp, s->p, s->stream));
+    } else
+#endif
+    {
+        WF_LAUNCH(s, WF_K_PRHS,
+                  wf_launch_pressure_rhs_fx(s->c, s->sp, ys, yn, s->p, form, P.pressure_solver_tol, s->press_rtol,
+                                            chk, max_iter, s->stream));
+        WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 1, s->sp.nz - 1, -1, 1, s->stream));
+        WF_LAUNCH(s, WF_K_THOMAS, wf_launch_thomas(s->sp, s->stream));
+        WF_LAUNCH(s, WF_K_PFY, wf_launch_fy(s->sp, s->F, sstride, 0, s->sp.nz, +1, 1, s->stream));
+        WF_LAUNCH(s, WF_K_PINV, wf_launch_inverse_fx(s->c, s->sp, s->p, s->stream));
+    }
     if (last)
         WF_LAUNCH(s, WF_K_OTHER,
                   wf_launch_iter_check(s->sp, P.pressure_solver_tol, s->press_rtol, m, max_iter, s->stream));
@@ -1229,7 +1278,7 @@ static bool ens_same_class(const Solver *a, const Solver *b) {
            a->P.variable_density == b->P.variable_density && wf_max_iter(a->P) == wf_max_iter(b->P) &&
            x.nx == y.nx && x.ny == y.ny && x.nz == y.nz && x.hx == y.hx && x.ldj == y.ldj &&
            x.fx_pairs == y.fx_pairs && x.fy_cols == y.fy_cols && x.ngroups == y.ngroups && x.npmax == y.npmax &&
-           x.thomas_lc == y.thomas_lc;
+           x.thomas_lc == y.thomas_lc && x.pl == y.pl && x.pl_nt == y.pl_nt;
 }
 
 /* Size classes (in order of first appearance) and the pressure operand
@@ -1430,11 +1479,20 @@ static int ens_pressure_class(Ensemble *e, int par, int q, hipStream_t st) {
     const long sstride = (long)sp.hx * sp.ldj;
     for (int m = 0; m < e->budget && m < max_iter; m++) {
         const int form = (m > 0) ? WF_F_ITER : (s0->P.variable_density ? WF_F_FIRST : WF_F_CONST);
-        WF_HIP(wf_launch_pressure_rhs_fx_batch(sp, tab, nm, form, m - 1, st));
-        WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 1, sp.nz - 1, -1, 1, st));
-        WF_HIP(wf_launch_thomas_batch(sp, tab, nm, st));
-        WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 0, sp.nz, +1, 1, st));
-        WF_HIP(wf_launch_inverse_fx_batch(sp, tab, nm, st));
+#if !WF_MIXED
+        if (sp.pl) {
+            WF_HIP(wf_launch_pl_rhs_batch(sp, tab, nm, form, m - 1, st));
+            WF_HIP(wf_launch_pl_solve_batch(sp, tab, nm, st));
+            WF_HIP(wf_launch_pl_inv_batch(sp, tab, nm, st));
+        } else
+#endif
+        {
+            WF_HIP(wf_launch_pressure_rhs_fx_batch(sp, tab, nm, form, m - 1, st));
+            WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 1, sp.nz - 1, -1, 1, st));
+            WF_HIP(wf_launch_thomas_batch(sp, tab, nm, st));
+            WF_HIP(wf_launch_fy_batch(sp, tab, nm, sstride, 0, sp.nz, +1, 1, st));
+            WF_HIP(wf_launch_inverse_fx_batch(sp, tab, nm, st));
+        }
         if (m + 1 >= e->budget || m + 1 >= max_iter) WF_HIP(wf_launch_iter_check_batch(tab, nm, m, st));
     }
     return WF_OK;
