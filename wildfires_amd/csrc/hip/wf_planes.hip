@@ -213,13 +213,13 @@ __device__ __forceinline__ void wf_pl_rhs_body(const WfConst &c, const WfSpectra
 }
 
 template <int MODE>
-__global__ __launch_bounds__(1024) void k_pl_rhs(WfConst c, WfSpectral sp, WfState Ys, WfState Yn, const wf_real *p,
+__global__ __launch_bounds__(512) void k_pl_rhs(WfConst c, WfSpectral sp, WfState Ys, WfState Yn, const wf_real *p,
                                                  double tol, double rtol, int check, int max_iter) {
     const int b = wf_checked_block(sp, tol, rtol, check, max_iter);
     if (b >= 0) wf_pl_rhs_body<MODE>(c, sp, Ys, Yn, p, b);
 }
 template <int MODE>
-__global__ __launch_bounds__(1024) void k_pl_rhs_batch(const WfPressItem *__restrict__ tab, int check) {
+__global__ __launch_bounds__(512) void k_pl_rhs_batch(const WfPressItem *__restrict__ tab, int check) {
     const WfPressItem it = wf_press_load(tab);
     const int b = wf_checked_block(it.sp, it.tol, it.rtol, check, it.max_iter);
     if (b >= 0) wf_pl_rhs_body<MODE>(it.c, it.sp, it.ys, it.yn, it.p, b);
@@ -713,8 +713,8 @@ __device__ __forceinline__ void wf_pl_inv_body(const WfConst &c, const WfSpectra
     }
     wf_block_max_store(dmax, &sp.pmax[blockIdx.x]);
 }
-__global__ __launch_bounds__(1024) void k_pl_inv(WfConst c, WfSpectral sp, wf_real *p) { wf_pl_inv_body(c, sp, p); }
-__global__ __launch_bounds__(1024) void k_pl_inv_batch(const WfPressItem *__restrict__ tab) {
+__global__ __launch_bounds__(512) void k_pl_inv(WfConst c, WfSpectral sp, wf_real *p) { wf_pl_inv_body(c, sp, p); }
+__global__ __launch_bounds__(512) void k_pl_inv_batch(const WfPressItem *__restrict__ tab) {
     const WfPressItem it = wf_press_load(tab);
     wf_pl_inv_body(it.c, it.sp, it.p);
 }
