@@ -15,10 +15,11 @@
  * The weight gradients are straight-through: the bf16 rounding of the
  * weights counts as the identity.
  *
- * Gradient kernel: one wavefront per workgroup; each pass takes 32 rows, in
- * two 16-row tiles for the forward products and as the K dimension of the
- * weight-gradient products.  Per-workgroup partial sums are reduced in a
- * fixed order, so a gradient is deterministic.
+ * Gradient kernel: each pass of a workgroup takes 32 rows, in two 16-row
+ * tiles for the forward products and as the K dimension of the
+ * weight-gradient products; each of its four wavefronts owns 16 of the 64
+ * hidden units.  Per-workgroup partial sums are reduced in a fixed order, so a
+ * gradient is deterministic.
  */
 #include <math.h>
 #include <stdint.h>
@@ -33,7 +34,7 @@ using namespace WF_NS; /* compiled once, in the FP64 namespace */
 #define WF_CLT_NP (WF_CL_NPARAMS + 1) /* gradient entries + the loss */
 #define WF_CLT_MAXWG 1024
 
-/* per-wavefront LDS of the trainer: activations and deltas of 32 rows in row
+/* per-workgroup LDS of the trainer: activations and deltas of 32 rows in row
  * ([row][unit]) and transposed ([unit][row]) order, bf16 */
 struct __attribute__((aligned(16))) WfClTrainLds {
     __bf16 a1s[32 * 64], a1t[64 * 32], a2s[32 * 64];
@@ -51,30 +52,33 @@ __device__ __forceinline__ float wf_cl_gelu_d(float h) {
 __host__ __device__ __forceinline__ bool wf_cl_trainable(int q) { return q >= WF_CL_W1 && q <= WF_CL_B3; }
 
 /* x: rows of 16 bf16 (12 normalised inputs, 4 zeros); t: targets nu / out_scale.
- * Rows [off, off + cnt); part: per workgroup WF_CLT_NP partial sums. */
-__global__ __launch_bounds__(64) void k_cl_grad(WfClosure cl, const wf_bf16x8 *w2bt, const __bf16 *x, const float *t,
-                                                long off, long cnt, float w, float *part) {
+ * Rows [off, off + cnt); part: per workgroup WF_CLT_NP partial sums.
+ * A batch of 8192 rows is one pass of 256 workgroups, so the kernel is as long
+ * as the chain of one pass: four exponentials and divisions per row and hidden
+ * unit.  With one wavefront per pass that chain covered all 64 units (22 us;
+ * 12 us with four wavefronts of 16 units each). */
+__global__ __launch_bounds__(256) void k_cl_grad(WfClosure cl, const wf_bf16x8 *w2bt, const __bf16 *x, const float *t,
+                                                 long off, long cnt, float w, float *part) {
     __shared__ WfClTrainLds L;
-    const int l = threadIdx.x, lr = l & 15, lg = l >> 4;
+    const int l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
+    const int nt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); /* the wavefront's units 16 nt .. 16 nt + 15 */
+    const int n = nt * 16 + lr;
     const float *prm = cl.prm;
     const wf_bf16x8 *W1 = cl.frag + WF_CL_FRAG_W1, *W2 = cl.frag + WF_CL_FRAG_W2, *W3 = cl.frag + WF_CL_FRAG_W3;
-    float w3b[4];
+    const wf_bf16x8 w1 = W1[nt * 64 + l], w2a = W2[(nt * 2) * 64 + l], w2b = W2[(nt * 2 + 1) * 64 + l];
+    const wf_bf16x8 w3a = W3[l], w3c = W3[64 + l], wta = w2bt[(nt * 2) * 64 + l], wtb = w2bt[(nt * 2 + 1) * 64 + l];
+    const float b1 = prm[WF_CL_B1 + n], b2 = prm[WF_CL_B2 + n], b3 = prm[WF_CL_B3];
+    const float w3b = (float)(__bf16)prm[WF_CL_W3 + n];
+    wf_f32x4 gW2[4], gW1 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) w3b[nt] = (float)(__bf16)prm[WF_CL_W3 + nt * 16 + lr];
-    wf_f32x4 gW2[4][4], gW1[4];
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        gW1[a] = wf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int b = 0; b < 4; b++) gW2[a][b] = wf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    float gw3[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0}, gb1[4] = {0, 0, 0, 0}, gb3 = 0.0f, loss = 0.0f;
+    for (int b = 0; b < 4; b++) gW2[b] = wf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float gw3 = 0.0f, gb2 = 0.0f, gb1 = 0.0f, gb3 = 0.0f, loss = 0.0f;
     const long ngroups = (cnt + 31) / 32;
     for (long grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
         const long base = off + grp * 32;
         const long last = off + cnt - 1;
         /* forward */
-        wf_f32x4 h1[2][4], h2[2][4];
+        wf_f32x4 h1[2], h2[2];
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
             long row = base + mt * 16 + lr;
@@ -83,90 +87,86 @@ __global__ __launch_bounds__(64) void k_cl_grad(WfClosure cl, const wf_bf16x8 *w
             if (lg < 2) a = *(const wf_bf16x8 *)&x[row * 16 + 8 * lg];
 #pragma unroll
             for (int j = 0; j < 8; j++)
-                if (lg < 2) L.xt[(8 * lg + j) * 32 + mt * 16 + lr] = a[j];
+                if (nt == 0 && lg < 2) L.xt[(8 * lg + j) * 32 + mt * 16 + lr] = a[j];
+            const wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w1, wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, W1[nt * 64 + l], wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
-                const int n = nt * 16 + lr;
-                const float b = prm[WF_CL_B1 + n];
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    h1[mt][nt][r] = d[r] + b;
-                    const __bf16 v = (__bf16)wf_cl_gelu(h1[mt][nt][r]);
-                    const int s = mt * 16 + 4 * lg + r;
-                    L.a1s[s * 64 + n] = v;
-                    L.a1t[n * 32 + s] = v;
-                }
+            for (int r = 0; r < 4; r++) {
+                h1[mt][r] = d[r] + b1;
+                const __bf16 v = (__bf16)wf_cl_gelu(h1[mt][r]);
+                const int s = mt * 16 + 4 * lg + r;
+                L.a1s[s * 64 + n] = v;
+                L.a1t[n * 32 + s] = v;
             }
         }
-        wf_cl_wave_sync();
+        __syncthreads();
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
             const wf_bf16x8 aa = *(const wf_bf16x8 *)&L.a1s[(mt * 16 + lr) * 64 + 8 * lg];
             const wf_bf16x8 ab = *(const wf_bf16x8 *)&L.a1s[(mt * 16 + lr) * 64 + 32 + 8 * lg];
+            wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa, w2a, wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, w2b, d, 0, 0, 0);
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa, W2[(nt * 2) * 64 + l], wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, W2[(nt * 2 + 1) * 64 + l], d, 0, 0, 0);
-                const int n = nt * 16 + lr;
-                const float b = prm[WF_CL_B2 + n];
+            for (int r = 0; r < 4; r++) {
+                h2[mt][r] = d[r] + b2;
+                L.a2s[(mt * 16 + 4 * lg + r) * 64 + n] = (__bf16)wf_cl_gelu(h2[mt][r]);
+            }
+        }
+        __syncthreads();
+        if (nt == 0) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    h2[mt][nt][r] = d[r] + b;
-                    L.a2s[(mt * 16 + 4 * lg + r) * 64 + n] = (__bf16)wf_cl_gelu(h2[mt][nt][r]);
+            for (int mt = 0; mt < 2; mt++) {
+                const wf_bf16x8 aa = *(const wf_bf16x8 *)&L.a2s[(mt * 16 + lr) * 64 + 8 * lg];
+                const wf_bf16x8 ab = *(const wf_bf16x8 *)&L.a2s[(mt * 16 + lr) * 64 + 32 + 8 * lg];
+                wf_f32x4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa, w3a, wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
+                z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, w3c, z, 0, 0, 0);
+                if (lr == 0) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int s = mt * 16 + 4 * lg + r;
+                        const long row = base + s;
+                        const float zv = z[r] + b3;
+                        const float e = (row <= last) ? wf_cl_softplus(zv) - t[row] : 0.0f;
+                        loss += w * e * e;
+                        const float dz = 2.0f * w * e * (1.0f / (1.0f + expf(-zv)));
+                        gb3 += dz;
+                        L.dz[s] = dz;
+                    }
                 }
             }
         }
-        wf_cl_wave_sync();
+        /* gelu' of both layers does not wait for dz */
+        float g1[2][4], g2[2][4];
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            const wf_bf16x8 aa = *(const wf_bf16x8 *)&L.a2s[(mt * 16 + lr) * 64 + 8 * lg];
-            const wf_bf16x8 ab = *(const wf_bf16x8 *)&L.a2s[(mt * 16 + lr) * 64 + 32 + 8 * lg];
-            wf_f32x4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa, W3[l], wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
-            z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab, W3[64 + l], z, 0, 0, 0);
-            if (lr == 0) {
+        for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int s = mt * 16 + 4 * lg + r;
-                    const long row = base + s;
-                    const float zv = z[r] + prm[WF_CL_B3];
-                    const float e = (row <= last) ? wf_cl_softplus(zv) - t[row] : 0.0f;
-                    loss += w * e * e;
-                    const float dz = 2.0f * w * e * (1.0f / (1.0f + expf(-zv)));
-                    gb3 += dz;
-                    L.dz[s] = dz;
-                }
+            for (int r = 0; r < 4; r++) {
+                g1[mt][r] = wf_cl_gelu_d(h1[mt][r]);
+                g2[mt][r] = wf_cl_gelu_d(h2[mt][r]);
             }
-        }
-        wf_cl_wave_sync();
+        __syncthreads();
         /* backward: output layer and second hidden layer */
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                const int n = nt * 16 + lr;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int s = mt * 16 + 4 * lg + r;
-                    const float dz = L.dz[s];
-                    gw3[nt] += dz * (float)L.a2s[s * 64 + n];
-                    const float d = dz * w3b[nt] * wf_cl_gelu_d(h2[mt][nt][r]);
-                    gb2[nt] += d;
-                    const __bf16 db = (__bf16)d;
-                    L.dh2s[s * 64 + n] = db;
-                    L.dh2t[n * 32 + s] = db;
-                }
+            for (int r = 0; r < 4; r++) {
+                const int s = mt * 16 + 4 * lg + r;
+                const float dz = L.dz[s];
+                gw3 += dz * (float)L.a2s[s * 64 + n];
+                const float d = dz * w3b * g2[mt][r];
+                gb2 += d;
+                const __bf16 db = (__bf16)d;
+                L.dh2s[s * 64 + n] = db;
+                L.dh2t[n * 32 + s] = db;
             }
         }
-        wf_cl_wave_sync();
-        /* dW2 += bf16(dh2)^T a1 over the 32 rows */
-#pragma unroll
-        for (int mo = 0; mo < 4; mo++) {
-            const wf_bf16x8 A = *(const wf_bf16x8 *)&L.dh2t[(mo * 16 + lr) * 32 + 8 * lg];
+        __syncthreads();
+        /* dW2 += bf16(dh2)^T a1 over the 32 rows (the wavefront's 16 rows of dW2) */
+        {
+            const wf_bf16x8 A = *(const wf_bf16x8 *)&L.dh2t[n * 32 + 8 * lg];
 #pragma unroll
             for (int ki = 0; ki < 4; ki++) {
                 const wf_bf16x8 B = *(const wf_bf16x8 *)&L.a1t[(ki * 16 + lr) * 32 + 8 * lg];
-                gW2[mo][ki] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, gW2[mo][ki], 0, 0, 0);
+                gW2[ki] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, gW2[ki], 0, 0, 0);
             }
         }
         /* da1 = bf16(dh2) W2, then dh1 */
@@ -174,121 +174,117 @@ __global__ __launch_bounds__(64) void k_cl_grad(WfClosure cl, const wf_bf16x8 *w
         for (int mt = 0; mt < 2; mt++) {
             const wf_bf16x8 Aa = *(const wf_bf16x8 *)&L.dh2s[(mt * 16 + lr) * 64 + 8 * lg];
             const wf_bf16x8 Ab = *(const wf_bf16x8 *)&L.dh2s[(mt * 16 + lr) * 64 + 32 + 8 * lg];
+            wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Aa, wta, wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ab, wtb, d, 0, 0, 0);
 #pragma unroll
-            for (int ki = 0; ki < 4; ki++) {
-                wf_f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Aa, w2bt[(ki * 2) * 64 + l], wf_f32x4{0, 0, 0, 0}, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ab, w2bt[(ki * 2 + 1) * 64 + l], d, 0, 0, 0);
-                const int k = ki * 16 + lr;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int s = mt * 16 + 4 * lg + r;
-                    const float dh = d[r] * wf_cl_gelu_d(h1[mt][ki][r]);
-                    gb1[ki] += dh;
-                    L.dh1t[k * 32 + s] = (__bf16)dh;
-                }
+            for (int r = 0; r < 4; r++) {
+                const int s = mt * 16 + 4 * lg + r;
+                const float dh = d[r] * g1[mt][r];
+                gb1 += dh;
+                L.dh1t[n * 32 + s] = (__bf16)dh;
             }
         }
-        wf_cl_wave_sync();
+        wf_cl_wave_sync(); /* dh1t: a wavefront reads the rows that it wrote */
         /* dW1 += bf16(dh1)^T x over the 32 rows (input columns 12..15 are zero) */
-        const wf_bf16x8 B = *(const wf_bf16x8 *)&L.xt[lr * 32 + 8 * lg];
-#pragma unroll
-        for (int mo = 0; mo < 4; mo++) {
-            const wf_bf16x8 A = *(const wf_bf16x8 *)&L.dh1t[(mo * 16 + lr) * 32 + 8 * lg];
-            gW1[mo] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, gW1[mo], 0, 0, 0);
+        {
+            const wf_bf16x8 B = *(const wf_bf16x8 *)&L.xt[lr * 32 + 8 * lg];
+            const wf_bf16x8 A = *(const wf_bf16x8 *)&L.dh1t[n * 32 + 8 * lg];
+            gW1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, gW1, 0, 0, 0);
         }
-        wf_cl_wave_sync(); /* this pass's LDS reads are done before the next pass writes */
+        __syncthreads(); /* this pass's LDS reads are done before the next pass writes */
     }
     /* partial sums of this workgroup */
     float *P = part + (long)blockIdx.x * WF_CLT_NP;
 #pragma unroll
-    for (int mo = 0; mo < 4; mo++) {
+    for (int r = 0; r < 4; r++) {
+        const int m = nt * 16 + 4 * lg + r;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int n = mo * 16 + 4 * lg + r;
-#pragma unroll
-            for (int ki = 0; ki < 4; ki++) P[WF_CL_W2 + n * 64 + ki * 16 + lr] = gW2[mo][ki][r];
-            if (lr < WF_CL_NIN) P[WF_CL_W1 + n * WF_CL_NIN + lr] = gW1[mo][r];
-        }
+        for (int ki = 0; ki < 4; ki++) P[WF_CL_W2 + m * 64 + ki * 16 + lr] = gW2[ki][r];
+        if (lr < WF_CL_NIN) P[WF_CL_W1 + m * WF_CL_NIN + lr] = gW1[r];
     }
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-        float a = gw3[nt], b = gb2[nt], c = gb1[nt];
-        a += __shfl_xor(a, 16, 64);
-        a += __shfl_xor(a, 32, 64);
-        b += __shfl_xor(b, 16, 64);
-        b += __shfl_xor(b, 32, 64);
-        c += __shfl_xor(c, 16, 64);
-        c += __shfl_xor(c, 32, 64);
-        if (lg == 0) {
-            P[WF_CL_W3 + nt * 16 + lr] = a;
-            P[WF_CL_B2 + nt * 16 + lr] = b;
-            P[WF_CL_B1 + nt * 16 + lr] = c;
-        }
+    gw3 += __shfl_xor(gw3, 16, 64);
+    gw3 += __shfl_xor(gw3, 32, 64);
+    gb2 += __shfl_xor(gb2, 16, 64);
+    gb2 += __shfl_xor(gb2, 32, 64);
+    gb1 += __shfl_xor(gb1, 16, 64);
+    gb1 += __shfl_xor(gb1, 32, 64);
+    if (lg == 0) {
+        P[WF_CL_W3 + n] = gw3;
+        P[WF_CL_B2 + n] = gb2;
+        P[WF_CL_B1 + n] = gb1;
     }
     for (int o = 32; o > 0; o >>= 1) {
         gb3 += __shfl_xor(gb3, o, 64);
         loss += __shfl_xor(loss, o, 64);
     }
-    if (l == 0) {
+    if (threadIdx.x == 0) {
         P[WF_CL_B3] = gb3;
         P[WF_CL_NPARAMS] = loss;
     }
 }
 
-/* grad[q] = sum over the nwg partials (trainable entries and the loss; 0 elsewhere) */
-__global__ void k_cl_reduce(const float *part, int nwg, float *grad) {
+/* Places of parameter q in the MFMA operands: the forward set of wf_closure.h
+ * and W2 for the da1 product (B[k = n][col = k_in] = W2[n][k_in], 4 column
+ * tiles x 2 K-steps), each an element of an operand of 8. */
+__device__ __forceinline__ void wf_cl_place(int q, float v, __bf16 *frag, __bf16 *w2bt) {
+    const __bf16 b = (__bf16)v;
+    if (q >= WF_CL_W1 && q < WF_CL_B1) {
+        const int n = (q - WF_CL_W1) / WF_CL_NIN, k = (q - WF_CL_W1) % WF_CL_NIN;
+        frag[(WF_CL_FRAG_W1 + (n >> 4) * 64 + (k >> 3) * 16 + (n & 15)) * 8 + (k & 7)] = b;
+    } else if (q >= WF_CL_W2 && q < WF_CL_B2) {
+        const int n = (q - WF_CL_W2) >> 6, k = (q - WF_CL_W2) & 63;
+        frag[(WF_CL_FRAG_W2 + ((n >> 4) * 2 + (k >> 5)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) * 8 + (k & 7)] = b;
+        w2bt[(((k >> 4) * 2 + (n >> 5)) * 64 + ((n & 31) >> 3) * 16 + (k & 15)) * 8 + (n & 7)] = b;
+    } else if (q >= WF_CL_W3 && q < WF_CL_B3) {
+        const int k = q - WF_CL_W3;
+        frag[(WF_CL_FRAG_W3 + (k >> 5) * 64 + ((k & 31) >> 3) * 16) * 8 + (k & 7)] = b;
+    }
+}
+/* the operands of an initial block (their other entries are 0) */
+__global__ void k_cl_place(const float *prm, __bf16 *frag, __bf16 *w2bt) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= WF_CLT_NP) return;
-    float s = 0.0f;
-    if (wf_cl_trainable(q) || q == WF_CL_NPARAMS)
-        for (int b = 0; b < nwg; b++) s += part[(long)b * WF_CLT_NP + q];
-    grad[q] = s;
+    if (q < WF_CL_NPARAMS) wf_cl_place(q, prm[q], frag, w2bt);
 }
 
-/* Adam on the trainable entries (bias-corrected, step >= 1) */
-__global__ void k_cl_adam(float *prm, float *m, float *v, const float *grad, float lr, float b1, float b2, float eps,
-                          int step) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= WF_CL_NPARAMS || !wf_cl_trainable(q)) return;
-    const float g = grad[q];
-    const float mq = b1 * m[q] + (1.0f - b1) * g;
-    const float vq = b2 * v[q] + (1.0f - b2) * g * g;
+/* grad[q] = sum over the nwg partials (trainable entries and the loss; 0
+ * elsewhere), in order.  Then, for a training step (step >= 1), Adam on the
+ * trainable entries (bias-corrected) and their places in the MFMA operands.
+ * One wavefront per workgroup, 64 partials of each entry in flight: the sum is
+ * a chain of additions, but its loads are independent (one load at a time in
+ * 20 workgroups took 58 us for 256 partials; with the update and the
+ * operands as launches of their own a step of 8192 rows took 90 us, now 20). */
+#define WF_CLT_RED 64
+__global__ __launch_bounds__(64) void k_cl_update(const float *part, int nwg, float *grad, float *prm, float *m,
+                                                  float *v, __bf16 *frag, __bf16 *w2bt, float lr, float b1, float b2,
+                                                  float eps, int step) {
+    const int q = blockIdx.x * 64 + threadIdx.x;
+    if (q >= WF_CLT_NP) return;
+    float s = 0.0f;
+    if (wf_cl_trainable(q) || q == WF_CL_NPARAMS) {
+        for (int b0 = 0; b0 < nwg; b0 += WF_CLT_RED) {
+            float a[WF_CLT_RED];
+#pragma unroll
+            for (int u = 0; u < WF_CLT_RED; u++) a[u] = part[(long)min(b0 + u, nwg - 1) * WF_CLT_NP + q];
+            if (b0 + WF_CLT_RED <= nwg) {
+#pragma unroll
+                for (int u = 0; u < WF_CLT_RED; u++) s += a[u];
+            } else {
+#pragma unroll
+                for (int u = 0; u < WF_CLT_RED; u++)
+                    if (b0 + u < nwg) s += a[u];
+            }
+        }
+    }
+    grad[q] = s;
+    if (step < 1 || q >= WF_CL_NPARAMS || !wf_cl_trainable(q)) return;
+    const float mq = b1 * m[q] + (1.0f - b1) * s;
+    const float vq = b2 * v[q] + (1.0f - b2) * s * s;
     m[q] = mq;
     v[q] = vq;
     const float mh = mq / (1.0f - powf(b1, (float)step)), vh = vq / (1.0f - powf(b2, (float)step));
-    prm[q] -= lr * mh / (sqrtf(vh) + eps);
-}
-
-/* The MFMA B fragments of prm (the forward set of wf_closure.h, and W2 for
- * the da1 product: B[k = n][col = k_in] = W2[n][k_in], 4 column tiles x 2 K-steps). */
-__global__ void k_cl_frags(const float *prm, wf_bf16x8 *frag, wf_bf16x8 *w2bt) {
-    const int l = threadIdx.x & 63, f = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int lr = l & 15, lg = l >> 4;
-    wf_bf16x8 o;
-    if (f < 4) { /* W1, output tile f */
-        const int n = f * 16 + lr;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int k = 8 * lg + j;
-            o[j] = (__bf16)((k < WF_CL_NIN) ? prm[WF_CL_W1 + n * WF_CL_NIN + k] : 0.0f);
-        }
-        frag[WF_CL_FRAG_W1 + f * 64 + l] = o;
-    } else if (f < 12) { /* W2, output tile nt, K-step ks */
-        const int nt = (f - 4) >> 1, ks = (f - 4) & 1, n = nt * 16 + lr;
-#pragma unroll
-        for (int j = 0; j < 8; j++) o[j] = (__bf16)prm[WF_CL_W2 + n * WF_CL_NH + ks * 32 + 8 * lg + j];
-        frag[WF_CL_FRAG_W2 + (f - 4) * 64 + l] = o;
-    } else if (f < 14) { /* w3 as column 0 */
-        const int ks = f - 12;
-#pragma unroll
-        for (int j = 0; j < 8; j++) o[j] = (__bf16)((lr == 0) ? prm[WF_CL_W3 + ks * 32 + 8 * lg + j] : 0.0f);
-        frag[WF_CL_FRAG_W3 + ks * 64 + l] = o;
-    } else if (f < 22) { /* W2 for da1: column tile ki, K-step ks */
-        const int ki = (f - 14) >> 1, ks = (f - 14) & 1, k = ki * 16 + lr;
-#pragma unroll
-        for (int j = 0; j < 8; j++) o[j] = (__bf16)prm[WF_CL_W2 + (ks * 32 + 8 * lg + j) * WF_CL_NH + k];
-        w2bt[(f - 14) * 64 + l] = o;
-    }
+    const float pq = prm[q] - lr * mh / (sqrtf(vh) + eps);
+    prm[q] = pq;
+    wf_cl_place(q, pq, frag, w2bt);
 }
 
 /* ---------------------------------------------------------------- C-ABI ---- */
@@ -308,20 +304,16 @@ struct wf_closure_trainer {
         if (e_ != hipSuccess) return wf_set_error(WF_E_DEVICE, hipGetErrorString(e_));           \
     } while (0)
 
-static int wf_clt_frags(wf_closure_trainer *T) {
-    hipLaunchKernelGGL(k_cl_frags, dim3(22), dim3(64), 0, 0, T->prm, T->frag, T->w2bt);
-    WF_CLT_HIP(hipGetLastError());
-    return WF_OK;
-}
-
-/* one gradient over rows [off, off + cnt) with weight w into T->grad */
-static int wf_clt_grad(wf_closure_trainer *T, long off, long cnt, float w) {
+/* one gradient over rows [off, off + cnt) with weight w into T->grad and, for
+ * training step `step` (0: none), the Adam step with it */
+static int wf_clt_grad(wf_closure_trainer *T, long off, long cnt, float w, float lr, int step) {
     const long groups = (cnt + 31) / 32;
     const int nwg = (int)((groups < WF_CLT_MAXWG) ? groups : WF_CLT_MAXWG);
-    hipLaunchKernelGGL(k_cl_grad, dim3(nwg), dim3(64), 0, 0, WfClosure{T->prm, T->frag}, T->w2bt, T->x, T->t, off,
+    hipLaunchKernelGGL(k_cl_grad, dim3(nwg), dim3(256), 0, 0, WfClosure{T->prm, T->frag}, T->w2bt, T->x, T->t, off,
                        cnt, w, T->part);
     WF_CLT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_cl_reduce, dim3((WF_CLT_NP + 255) / 256), dim3(256), 0, 0, T->part, nwg, T->grad);
+    hipLaunchKernelGGL(k_cl_update, dim3((WF_CLT_NP + 63) / 64), dim3(64), 0, 0, T->part, nwg, T->grad, T->prm, T->m,
+                       T->v, (__bf16 *)T->frag, (__bf16 *)T->w2bt, lr, 0.9f, 0.999f, 1e-8f, step);
     WF_CLT_HIP(hipGetLastError());
     return WF_OK;
 }
@@ -374,16 +366,20 @@ extern "C" int wf_closure_trainer_create(const float *params, long nparams, cons
     if (e == hipSuccess) e = hipMemcpy(T->prm, params, sizeof(float) * WF_CL_NPARAMS, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(T->m, 0, sizeof(float) * WF_CL_NPARAMS);
     if (e == hipSuccess) e = hipMemset(T->v, 0, sizeof(float) * WF_CL_NPARAMS);
+    if (e == hipSuccess) e = hipMemset(T->frag, 0, sizeof(wf_bf16x8) * WF_CL_NFRAG);
+    if (e == hipSuccess) e = hipMemset(T->w2bt, 0, sizeof(wf_bf16x8) * 8 * 64);
     if (e == hipSuccess) e = hipMemcpy(T->x, xb.data(), sizeof(uint16_t) * 16 * (size_t)n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(T->t, tb.data(), sizeof(float) * n, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         wf_closure_trainer_destroy(T);
         return wf_set_error(WF_E_DEVICE, hipGetErrorString(e));
     }
-    int rc = wf_clt_frags(T);
-    if (rc) {
+    hipLaunchKernelGGL(k_cl_place, dim3((WF_CL_NPARAMS + 63) / 64), dim3(64), 0, 0, T->prm, (__bf16 *)T->frag,
+                       (__bf16 *)T->w2bt);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
         wf_closure_trainer_destroy(T);
-        return rc;
+        return wf_set_error(WF_E_DEVICE, hipGetErrorString(e));
     }
     *out = T;
     return WF_OK;
@@ -393,7 +389,7 @@ extern "C" int wf_closure_trainer_gradient(wf_closure_trainer *T, long offset, l
                                            float *grad, double *loss) {
     if (T == NULL || grad == NULL || loss == NULL || offset < 0 || count <= 0 || offset + count > T->n)
         return wf_set_error(WF_E_ARG, "closure trainer: bad row range");
-    int rc = wf_clt_grad(T, offset, count, (float)weight);
+    int rc = wf_clt_grad(T, offset, count, (float)weight, 0.0f, 0);
     if (rc) return rc;
     std::vector<float> g(WF_CLT_NP);
     WF_CLT_HIP(hipMemcpy(g.data(), T->grad, sizeof(float) * WF_CLT_NP, hipMemcpyDeviceToHost));
@@ -408,14 +404,9 @@ extern "C" int wf_closure_trainer_train(wf_closure_trainer *T, int steps, long b
     long off = ((long)T->step * batch) % T->n;
     for (int s = 0; s < steps; s++) {
         if (off + batch > T->n) off = 0;
-        int rc = wf_clt_grad(T, off, batch, 1.0f / (float)batch);
+        int rc = wf_clt_grad(T, off, batch, 1.0f / (float)batch, (float)lr, T->step + 1);
         if (rc) return rc;
         T->step++;
-        hipLaunchKernelGGL(k_cl_adam, dim3((WF_CL_NPARAMS + 255) / 256), dim3(256), 0, 0, T->prm, T->m, T->v, T->grad,
-                           (float)lr, 0.9f, 0.999f, 1e-8f, T->step);
-        WF_CLT_HIP(hipGetLastError());
-        rc = wf_clt_frags(T);
-        if (rc) return rc;
         off += batch;
     }
     if (last_loss) {
