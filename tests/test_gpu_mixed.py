@@ -129,3 +129,23 @@ def test_mixed_flat64_1000_steps_small_fields(flat64_1000, name):
     if errs[name] > 1e-4:
         pytest.xfail("%s: %.2e after 1000 steps (FP32 rounding of the stored state at the velocity scale)"
                      % (name, errs[name]))
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(31, 36, 9), (22, 58, 8), (9, 127, 7), (148, 12, 9), (319, 14, 8), (16, 330, 7)])
+def test_mixed_run_time_lengths_close_to_fp64(tmp_path, monkeypatch, nx, ny, nz):
+    """Run-time transform stages of the mixed form: radices 2, 3, 4, 5, 7 and
+    11 to 83 in x and y, lengths with two and with four row pairs per
+    workgroup.  Four solves of the iteration within 2e-5 of FP64, the bound of
+    the other FP32 transform test: FP32 arithmetic alone."""
+    from oracle import oracle
+    from wildfires_amd import api
+    prm = make_params(tmp_path, "small_flat", Nx=nx, Ny=ny, Nz=nz, x_max=2.0 * (nx - 1), y_max=2.0 * (ny - 1),
+                      z_max=0.5 * (nz - 1), pressure_solver_iter=4)
+    y, p = perturbed_state(prm)
+    y1 = y + prm.p.dt * oracle.Oracle(prm.ptr).phi(y)
+    monkeypatch.setenv("WF_MIXED_PRESSURE_RTOL", "0")
+    pm, _, im = api.Solver(prm, "mixed").pressure(y1, y, p)
+    pd, _, idd = api.Solver(prm, "fp64").pressure(y1, y, p)
+    print("%dx%dx%d mixed vs fp64 %.3e" % (nx, ny, nz, rel_l2(pm, pd)), flush=True)
+    assert rel_l2(pm, pd) <= 2e-5
+    assert im == idd

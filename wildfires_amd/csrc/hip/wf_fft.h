@@ -3,12 +3,12 @@
  *
  * Lengths 63 and 255 (the 64- and 256-node grids) use a two-factor register
  * transform (below).  Any other length runs a mixed-radix Stockham transform
- * in LDS with run-time radices: stage with radix R after radices of product
+ * in LDS with run-time radices (wf_lds_fft): stage with radix R after radices of product
  * Ns (natural order, decimation in time): butterfly j in [0, n/R) reads
  * in[j + r n/R], r < R, and writes out[(j/Ns) Ns R + j%Ns + q Ns], q < R, with
- *   out = sum_r W_{Ns R}^{r (j%Ns + q Ns)} in[j + r n/R],  W_m = exp(sign 2 pi i / m),
- * one output element per thread.  wf_stockham_output is host/device-neutral so
- * the CPU check of the plan runs the same indexing.
+ *   out = sum_r W_{Ns R}^{r (j%Ns + q Ns)} in[j + r n/R],  W_m = exp(sign 2 pi i / m).
+ * wf_stockham_output states one output element of a stage; it is
+ * host/device-neutral, and the CPU check of the plan runs it.
  */
 #ifndef WF_FFT_H
 #define WF_FFT_H
@@ -95,10 +95,110 @@ __device__ __forceinline__ wfc wf_cmul(wfc a, wfc b) {
     return r;
 }
 
-/* One Stockham stage of radix R after radices of product NS over `nseq`
- * sequences of length N (same mathematics as wf_stockham_output).  Radices up
- * to 8 run one butterfly per thread with its R values in registers; larger
- * prime radices run one output per thread to keep the workgroup busy. */
+/* Quotients by a run-time divisor d through its reciprocal rounded up (exact
+ * for t < 2^16, d <= 2^10: t (2^32/d + 1) < 2^32 (t/d + 1/d)). */
+struct WfDiv {
+    unsigned m;
+    int d;
+    __device__ __forceinline__ explicit WfDiv(int div) : m(0xffffffffu / (unsigned)div + 1u), d(div) {}
+    __device__ __forceinline__ int operator()(int t) const { return (d == 1) ? t : (int)__umulhi((unsigned)t, m); }
+};
+
+/* Run-time Stockham stages, wf_stockham_output's terms in its order.  What
+ * bounds them is instructions: the index arithmetic of an output (five
+ * run-time divisions), and for every term two LDS reads and 8 separate
+ * roundings.  So a small radix takes a whole butterfly per thread (its R inputs
+ * read once, one set of indices for R outputs), and the others WF_RT_SEQ
+ * sequences per thread, which share indices and twiddles (two measured best:
+ * four leave too few threads, 32 us against 24 for the x pass of length 200).
+ * The term r = 0 has the factor (1, 0) and starts the sum.  FP32, us per pass,
+ * one output per thread before: y of length 150 at 201x151x81 30 -> 20, x of
+ * length 200 35 -> 24 and 32 -> 21; length 199 (prime) at 200x200x90 y 206 ->
+ * 132, x 166 -> 136. */
+template <int R>
+__device__ __forceinline__ void wf_rt_butterfly(const wfc *a, wfc *b, int n, int nseq, int Ns, const wfc *tw) {
+    const int m = n / R, scale = m / Ns;
+    const WfDiv by_m(m), by_ns(Ns);
+    for (int t = threadIdx.x; t < m * nseq; t += blockDim.x) {
+        const int s = by_m(t), j = t - s * m, jq = by_ns(j), kq = j - jq * Ns;
+        const wfc *in = a + s * n + j;
+        wfc *out = b + s * n + jq * Ns * R + kq;
+        wfc x[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) x[r] = in[r * m];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            const int step = kq * scale + q * m;
+            wfc acc = x[0];
+            int e = 0;
+#pragma unroll
+            for (int r = 1; r < R; r++) {
+                e += step;
+                e = (e >= n) ? e - n : e;
+                const wfc w = tw[e];
+                acc.re += w.re * x[r].re - w.im * x[r].im;
+                acc.im += w.re * x[r].im + w.im * x[r].re;
+            }
+            out[q * Ns] = acc;
+        }
+    }
+}
+#define WF_RT_SEQ 2
+__device__ __forceinline__ void wf_rt_outputs(const wfc *a, wfc *b, int n, int nseq, int R, int Ns, const wfc *tw) {
+    constexpr int S = WF_RT_SEQ;
+    const int m = n / R, scale = m / Ns;
+    const WfDiv by_n(n), by_ns(Ns), by_r(R);
+    for (int t = threadIdx.x; t < n * (nseq / S); t += blockDim.x) {
+        const int sg = by_n(t), o = t - sg * n;
+        const int rest = by_ns(o), kq = o - rest * Ns, jq = by_r(rest), q = rest - jq * R;
+        const wfc *in = a + sg * S * n + jq * Ns + kq;
+        const int step = kq * scale + q * m;
+        wfc acc[S];
+#pragma unroll
+        for (int s = 0; s < S; s++) acc[s] = in[s * n];
+        int e = 0;
+#pragma unroll 4
+        for (int r = 1; r < R; r++) {
+            e += step;
+            e = (e >= n) ? e - n : e;
+            in += m;
+            const wfc w = tw[e];
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const wfc x = in[s * n];
+                acc[s].re += w.re * x.re - w.im * x.im;
+                acc[s].im += w.re * x.im + w.im * x.re;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < S; s++) b[(sg * S + s) * n + o] = acc[s];
+    }
+}
+/* One full FFT of `nseq` sequences (a multiple of WF_RT_SEQ) of run-time
+ * length n held in LDS (a -> b -> a ...), for lengths without a compile-time
+ * plan.  Returns the buffer that holds the result. */
+__device__ __forceinline__ wfc *wf_lds_fft(wfc *a, wfc *b, int n, int nseq, const int *rad, const wfc *tw) {
+    int Ns = 1;
+    for (int p = 0; p < WF_MAX_RADICES; p++) {
+        const int R = rad[p];
+        if (R == 0) break;
+        switch (R) {
+            case 2: wf_rt_butterfly<2>(a, b, n, nseq, Ns, tw); break;
+            case 3: wf_rt_butterfly<3>(a, b, n, nseq, Ns, tw); break;
+            case 4: wf_rt_butterfly<4>(a, b, n, nseq, Ns, tw); break;
+            case 5: wf_rt_butterfly<5>(a, b, n, nseq, Ns, tw); break;
+            case 7: wf_rt_butterfly<7>(a, b, n, nseq, Ns, tw); break;
+            default: wf_rt_outputs(a, b, n, nseq, R, Ns, tw); break;
+        }
+        __syncthreads();
+        wfc *tmp = a;
+        a = b;
+        b = tmp;
+        Ns *= R;
+    }
+    return a;
+}
+
 /* ------------------------------------------------------------------------
  * Compile-time plans for the transform lengths of the supported grids.
  * The radix sequence of N is the one the host factoriser produces (4s, then

@@ -146,6 +146,8 @@ struct WfIterCtl {
 #define WF_FX_PAIRS 4
 #endif
 __host__ __device__ constexpr int wf_pairs_for(int n) { return (n <= 300) ? WF_FX_PAIRS : 2; }
+/* lengths with a compile-time plan */
+__host__ __device__ constexpr bool wf_planned(int n) { return n == 63 || n == 127 || n == 255 || n == 511; }
 #define WF_FY_COLS 4
 /* kx columns per workgroup of the in-place y-transform (lengths without a
  * two-factor plan).  Batched launches (many members, workgroups to spare) of

@@ -30,36 +30,26 @@
 
 namespace WF_NS {
 
-/* One full FFT of `nseq` sequences of run-time length n held in LDS
- * (a -> b -> a ...), for lengths without a compile-time plan.  Returns the
- * buffer that holds the result. */
-__device__ wfc *wf_lds_fft(wfc *a, wfc *b, int n, int nseq, const int *rad, const wfc *tw) {
-    int Ns = 1;
-    for (int p = 0; p < WF_MAX_RADICES; p++) {
-        int R = rad[p];
-        if (R == 0) break;
-        for (int t = threadIdx.x; t < n * nseq; t += blockDim.x) {
-            int s = t / n, o = t - s * n;
-            b[s * n + o] = wf_stockham_output(a + s * n, n, R, Ns, tw, o);
-        }
-        __syncthreads();
-        wfc *tmp = a;
-        a = b;
-        b = tmp;
-        Ns *= R;
-    }
-    return a;
-}
-
-/* Transform of the NSEQ sequences in buf (compile-time plan when N > 0, else
+/* Row pairs of an x-transform workgroup compiled for length NX, and the most
+ * elements a thread of it takes.  NX = 0 and -1 are the run-time lengths up
+ * to 300 and above. */
+#define WF_NX_SHORT 300
+template <int NX>
+struct WfFx {
+    static constexpr int LEN = (NX > 0) ? NX : (NX == 0) ? WF_NX_SHORT : 1024;
+    static constexpr int PAIRS = wf_pairs_for(LEN);
+    static constexpr int PER = (PAIRS * LEN + WF_NT - 1) / WF_NT;
+};
+/* Transform of the PAIRS sequences in buf (compile-time plan when NX > 0, else
  * the run-time radices with scratch buffer bufb).  Returns the result buffer. */
-template <int N, int NSEQ>
-__device__ __forceinline__ wfc *wf_transform(wfc *buf, wfc *bufb, int n, int nseq, const int *rad, const wfc *tw) {
-    if constexpr (N > 0) {
-        wf_fft_ip<N, NSEQ, WF_NT>(buf, tw);
+template <int NX>
+__device__ __forceinline__ wfc *wf_transform(wfc *buf, wfc *bufb, int n, const int *rad, const wfc *tw) {
+    constexpr int PAIRS = WfFx<NX>::PAIRS;
+    if constexpr (NX > 0) {
+        wf_fft_ip<NX, PAIRS, WF_NT>(buf, tw);
         return buf;
     } else {
-        return wf_lds_fft(buf, bufb, n, nseq, rad, tw);
+        return wf_lds_fft(buf, bufb, n, PAIRS, rad, tw);
     }
 }
 
@@ -98,55 +88,38 @@ __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectra
     if (MODE != WF_F_TOP && sp.ctl->done) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
-    constexpr int PAIRS = (NX > 0) ? wf_pairs_for(NX) : 0;
+    constexpr int PAIRS = WfFx<NX>::PAIRS, PER = WfFx<NX>::PER;
     const int nx = (NX > 0) ? NX : sp.nx;
-    const int pairs = (NX > 0) ? PAIRS : sp.fx_pairs;
     const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
-    wfc *tw = smem, *bufa = smem + nx, *bufb = bufa + pairs * nx;
+    wfc *tw = smem, *bufa = smem + nx, *bufb = bufa + PAIRS * nx;
     int g, ks;
     wf_tile_decode_at(block, nblocks, sp.ngroups, (MODE == WF_F_TOP) ? 1 : sp.nz - 1, &g, &ks);
     const int k = (MODE == WF_F_TOP) ? c.Nz - 1 : 1 + ks;
-    const int j0 = 2 * g * pairs;
+    const int j0 = 2 * g * PAIRS;
     for (int t = threadIdx.x; t < nx; t += blockDim.x) tw[t] = *(const wfc *)&sp.twx[t];
-    if (NX == 0 && threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
-    if constexpr (NX > 0 && MODE != WF_F_FIRST) {
-        /* one row pair per batch: both cells' loads unconditional (indices
-         * clamped to a valid node, padding results dropped), so a batch is
-         * one basic block with all 28 loads in flight; the scheduling
-         * barrier keeps the batches apart, which bounds the registers */
-        constexpr int PER = (PAIRS * NX + WF_NT - 1) / WF_NT;
+    if (NX <= 0 && threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
+    const WfDiv by_nx(nx);
+    /* one row pair per batch: both cells' loads unconditional (indices clamped
+     * to a valid node, padding results dropped), so a batch is one basic block
+     * with all 28 loads in flight; the scheduling barrier keeps the batches
+     * apart, which bounds the registers */
 #pragma unroll
-        for (int pi = 0; pi < PER; pi++) {
-            const int t = threadIdx.x + pi * WF_NT;
-            const int tc = (t < PAIRS * NX) ? t : PAIRS * NX - 1;
-            const int s = tc / NX, i = tc - s * NX;
+    for (int pi = 0; pi < PER; pi++) {
+        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
+        const int t = threadIdx.x + pi * WF_NT;
+        if constexpr (MODE != WF_F_FIRST) {
+            const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
+            const int s = (NX > 0) ? tc / nx : by_nx(tc), i = tc - s * nx;
             const int ja = j0 + 2 * s, jb = ja + 1;
             const wf_real fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (ja < ny) ? ja : ny - 1, k);
             const wf_real fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (jb < ny) ? jb : ny - 1, k);
-            if (t < PAIRS * NX) {
+            if (t < PAIRS * nx) {
                 bufa[t].re = (ja < ny) ? fa : WR(0.0);
                 bufa[t].im = (jb < ny) ? fb : WR(0.0);
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-    } else if constexpr (NX > 0) {
-        constexpr int PER = (PAIRS * NX + WF_NT - 1) / WF_NT;
-#pragma unroll
-        for (int pi = 0; pi < PER; pi++) {
-            const int t = threadIdx.x + pi * WF_NT;
-            if (t < PAIRS * NX) {
-                const int s = t / NX, i = t - s * NX;
-                const int ja = j0 + 2 * s, jb = ja + 1;
-                wf_real fa = WR(0.0), fb = WR(0.0);
-                if (ja < ny) fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, ja, k);
-                if (jb < ny) fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, jb, k);
-                bufa[t].re = fa;
-                bufa[t].im = fb;
-            }
-        }
-    } else {
-        for (int t = threadIdx.x; t < pairs * nx; t += blockDim.x) {
-            const int s = t / nx, i = t - s * nx;
+        } else if (t < PAIRS * nx) {
+            const int s = (NX > 0) ? t / nx : by_nx(t), i = t - s * nx;
             const int ja = j0 + 2 * s, jb = ja + 1;
             wf_real fa = WR(0.0), fb = WR(0.0);
             if (ja < ny) fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, ja, k);
@@ -156,9 +129,9 @@ __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectra
         }
     }
     __syncthreads();
-    wfc *res = wf_transform<NX, PAIRS>(bufa, bufb, nx, pairs, rad, tw);
+    wfc *res = wf_transform<NX>(bufa, bufb, nx, rad, tw);
     wf_real2 *dst = (MODE == WF_F_TOP) ? sp.Ptop : sp.F + (long)k * hx * ldj;
-    const int rows = 2 * pairs;
+    constexpr int rows = 2 * PAIRS;
     for (int t = threadIdx.x; t < rows * hx; t += blockDim.x) {
         const int jl = t % rows, r = t / rows;
         const int j = j0 + jl;
@@ -262,20 +235,24 @@ __device__ __forceinline__ void wf_fy_body(const WfSpectral &sp, wf_real2 *buf, 
             tw[t].im = (sign > 0) ? -w.y : w.y;
         }
         if (threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.rady[threadIdx.x];
-        for (int t = threadIdx.x; t < cols * ny; t += blockDim.x) {
-            const int cc = t / ny, jj = t - cc * ny;
-            wfc v = {WR(0.0), WR(0.0)};
-            if (r0 + cc < hx) {
-                wf_real2 x = base[(long)(r0 + cc) * ldj + jj];
-                v.re = x.x;
-                v.im = x.y;
+        const WfDiv by_ny(ny);
+        constexpr int B = 4;
+        for (int t0 = threadIdx.x; t0 < cols * ny; t0 += B * WF_NT) {
+            wf_real2 x[B];
+#pragma unroll
+            for (int u = 0; u < B; u++) {
+                const int t = min(t0 + u * WF_NT, cols * ny - 1);
+                const int cc = by_ny(t), jj = t - cc * ny;
+                x[u] = base[(long)min(r0 + cc, hx - 1) * ldj + jj];
             }
-            bufa[t] = v;
+#pragma unroll
+            for (int u = 0; u < B; u++)
+                if (t0 + u * WF_NT < cols * ny) bufa[t0 + u * WF_NT] = wfc{x[u].x, x[u].y};
         }
         __syncthreads();
         wfc *res = wf_lds_fft(bufa, bufb, ny, cols, rad, tw);
         for (int t = threadIdx.x; t < cols * ny; t += blockDim.x) {
-            const int cc = t / ny, jj = t - cc * ny;
+            const int cc = by_ny(t), jj = t - cc * ny;
             if (r0 + cc < hx) base[(long)(r0 + cc) * ldj + jj] = wf_make2(res[t].re, res[t].im);
         }
     }
@@ -603,71 +580,36 @@ __global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) __attribute__((amdgpu_wa
  * workgroup refreshes the periodic copies on the top plane, which the solve
  * never writes on unique nodes. */
 
-/* new value pv of node (i, j, k) and of its periodic duplicates, with the
- * running max |p_new - p_old| */
-__device__ __forceinline__ void wf_put_p_old(const WfConst &c, wf_real *p, int i, int j, int k, wf_real pv, wf_real pold,
-                                             double &dmax, double &pabs) {
-    const long q = wf_q(c, i, j, k);
-    const double d = (double)fabs(pv - pold);
-    dmax = (d > dmax) ? d : dmax;
-    if constexpr (WF_MIXED) {
-        const double a = (double)fabs(pv);
-        pabs = (a > pabs) ? a : pabs;
-    }
-    p[q] = pv;
-    if (i == 0) { /* duplicate column i = Nx-1 */
-        const long qd = wf_q(c, c.Nx - 1, j, k);
-        const double dd = (double)fabs(pv - p[qd]);
-        dmax = (dd > dmax) ? dd : dmax;
-        p[qd] = pv;
-    }
-    if (j == 0) { /* duplicate row j = Ny-1 */
-        const long qd = wf_q(c, i, c.Ny - 1, k);
-        const double dd = (double)fabs(pv - p[qd]);
-        dmax = (dd > dmax) ? dd : dmax;
-        p[qd] = pv;
-        if (i == 0) {
-            const long qc = wf_q(c, c.Nx - 1, c.Ny - 1, k);
-            const double dc = (double)fabs(pv - p[qc]);
-            dmax = (dc > dmax) ? dc : dmax;
-            p[qc] = pv;
-        }
-    }
-}
-__device__ __forceinline__ void wf_put_p(const WfConst &c, wf_real *p, int i, int j, int k, wf_real pv, double &dmax,
-                                         double &pabs) {
-    wf_put_p_old(c, p, i, j, k, pv, p[wf_q(c, i, j, k)], dmax, pabs);
-}
-
-/* Compile-time plan of P5: every global load (half spectra, the old p of the
+/* P5: every global load (half spectra, the old p of the
  * group's unique nodes and of their periodic duplicates) is issued before the
  * transform, unconditionally with clamped indices, so a workgroup waits for
  * one memory round trip; the stores of the duplicates use no branches inside
  * the main loop (column i = Nx-1 from threads 0 .. 2*PAIRS-1, row j = Ny-1 by
- * the group that holds j = 0).  The set of (node, new value) pairs, and so
- * the norm, is the one of wf_put_p. */
+ * the group that holds j = 0). */
 template <int NX>
-__device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpectral &sp, wf_real *p, wfc *smem,
-                                                  int g, int k, double &dmax, double &pabs) {
-    constexpr int PAIRS = wf_pairs_for(NX);
-    constexpr int PER = (PAIRS * NX + WF_NT - 1) / WF_NT;
-    constexpr int PERY = (NX + 1 + WF_NT - 1) / WF_NT; /* row j = Ny-1: i = 0 .. Nx-1 */
+__device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectral &sp, wf_real *p, wfc *smem,
+                                                  const int *rad, int g, int k, double &dmax, double &pabs) {
+    constexpr int PAIRS = WfFx<NX>::PAIRS, PER = WfFx<NX>::PER;
+    constexpr int PERY = (WfFx<NX>::LEN + 1 + WF_NT - 1) / WF_NT; /* row j = Ny-1: i = 0 .. Nx-1 */
+    const int nx = (NX > 0) ? NX : sp.nx;
+    const WfDiv by_nx(nx);
     const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
     const int j0 = 2 * g * PAIRS;
     const wf_real2 *src = sp.F + (long)k * hx * ldj;
-    const wf_real inv_scale = WR(1.0) / ((wf_real)NX * (wf_real)ny);
+    const wf_real inv_scale = WR(1.0) / ((wf_real)nx * (wf_real)ny);
     const int tid = threadIdx.x;
-    wfc *tw = smem, *buf = smem + NX;
+    wfc *tw = smem, *buf = smem + nx;
     /* loads: half spectra (thread t -> pair t % PAIRS, bin t / PAIRS, so
      * consecutive threads read consecutive ky of one kx column) */
     wf_real2 xa[PER], xb[PER];
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
+        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
         const int t = tid + pi * WF_NT;
-        const int tc = (t < PAIRS * NX) ? t : PAIRS * NX - 1;
+        const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
         const int s = tc % PAIRS, r = tc / PAIRS;
         const int ja = j0 + 2 * s, jb = ja + 1;
-        const int rr = (r >= hx) ? NX - r : r;
+        const int rr = (r >= hx) ? nx - r : r;
         xa[pi] = src[(long)rr * ldj + ((ja < ny) ? ja : ny - 1)];
         xb[pi] = src[(long)rr * ldj + ((jb < ny) ? jb : ny - 1)];
     }
@@ -675,9 +617,10 @@ __device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpec
     wf_real pa[PER], pb[PER];
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
+        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
         const int t = tid + pi * WF_NT;
-        const int tc = (t < PAIRS * NX) ? t : PAIRS * NX - 1;
-        const int s = tc / NX, i = tc - s * NX;
+        const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
+        const int s = (NX > 0) ? tc / nx : by_nx(tc), i = tc - s * nx;
         const int ja = j0 + 2 * s, jb = ja + 1;
         pa[pi] = p[wf_q(c, i, (ja < ny) ? ja : ny - 1, k)];
         pb[pi] = p[wf_q(c, i, (jb < ny) ? jb : ny - 1, k)];
@@ -691,20 +634,21 @@ __device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpec
 #pragma unroll
         for (int pi = 0; pi < PERY; pi++) {
             const int i = tid + pi * WF_NT;
-            pdy[pi] = p[wf_q(c, (i <= NX) ? i : NX, c.Ny - 1, k)];
+            pdy[pi] = p[wf_q(c, (i <= nx) ? i : nx, c.Ny - 1, k)];
         }
     }
-    for (int t = tid; t < NX; t += WF_NT) {
+    for (int t = tid; t < nx; t += WF_NT) {
         const wf_real2 w = sp.twx[t];
         tw[t].re = w.x;
         tw[t].im = -w.y;
     }
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
+        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
         const int t = tid + pi * WF_NT;
         const int s = t % PAIRS, r = t / PAIRS;
         const int ja = j0 + 2 * s, jb = ja + 1;
-        if (t < PAIRS * NX) {
+        if (t < PAIRS * nx) {
             wfc A = {WR(0.0), WR(0.0)}, B = {WR(0.0), WR(0.0)};
             if (ja < ny) {
                 A.re = xa[pi].x;
@@ -714,19 +658,20 @@ __device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpec
                     B.im = xb[pi].y;
                 }
             }
-            buf[s * NX + r] = wf_pack_pair(A, B, r >= hx);
+            buf[s * nx + r] = wf_pack_pair(A, B, r >= hx);
         }
     }
     __syncthreads();
-    wf_fft_ip<NX, PAIRS, WF_NT>(buf, tw);
+    buf = wf_transform<NX>(buf, buf + PAIRS * nx, nx, rad, tw);
     /* unique nodes */
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
+        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
         const int t = tid + pi * WF_NT;
-        const int s = t / NX, i = t - s * NX;
+        const int s = (NX > 0) ? t / nx : by_nx(t), i = t - s * nx;
         const int ja = j0 + 2 * s, jb = ja + 1;
-        if (t < PAIRS * NX) {
-            const wfc v = buf[s * NX + i];
+        if (t < PAIRS * nx) {
+            const wfc v = buf[s * nx + i];
             if (ja < ny) {
                 const wf_real pv = v.re * inv_scale;
                 const double d = (double)fabs(pv - pa[pi]);
@@ -745,7 +690,7 @@ __device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpec
     }
     /* duplicate column i = Nx-1 of rows j0 .. j0 + 2 PAIRS - 1 (value of i = 0) */
     if (tid < 2 * PAIRS && jr < ny) {
-        const wfc v = buf[(tid >> 1) * NX];
+        const wfc v = buf[(tid >> 1) * nx];
         const wf_real pv = ((tid & 1) ? v.im : v.re) * inv_scale;
         const double d = (double)fabs(pv - pdx);
         dmax = (d > dmax) ? d : dmax;
@@ -756,8 +701,8 @@ __device__ __forceinline__ void wf_inv_fx_planned(const WfConst &c, const WfSpec
 #pragma unroll
         for (int pi = 0; pi < PERY; pi++) {
             const int i = tid + pi * WF_NT;
-            if (i <= NX) {
-                const wf_real pv = buf[(i < NX) ? i : 0].re * inv_scale;
+            if (i <= nx) {
+                const wf_real pv = buf[(i < nx) ? i : 0].re * inv_scale;
                 const double d = (double)fabs(pv - pdy[pi]);
                 dmax = (d > dmax) ? d : dmax;
                 p[wf_q(c, i, c.Ny - 1, k)] = pv;
@@ -771,9 +716,6 @@ __device__ __forceinline__ void wf_inv_fx_body(const WfConst &c, const WfSpectra
     if (sp.ctl->done) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
-    const int nx = (NX > 0) ? NX : sp.nx;
-    const int pairs = sp.fx_pairs;
-    const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
     double dmax = 0.0, pabs = 0.0;
     if (blockIdx.x == gridDim.x - 1) {
         wf_top_duplicates(c, p, dmax);
@@ -787,48 +729,8 @@ __device__ __forceinline__ void wf_inv_fx_body(const WfConst &c, const WfSpectra
     /* the tiles are blocks 0 .. gridDim.x - 2 (the last block is the one above) */
     int g, k;
     wf_tile_decode_at((int)blockIdx.x, (int)gridDim.x - 1, sp.ngroups, sp.nz, &g, &k);
-    if constexpr (NX > 0) {
-        wf_inv_fx_planned<NX>(c, sp, p, smem, g, k, dmax, pabs);
-    } else {
-        const int j0 = 2 * g * pairs;
-        const wf_real2 *src = sp.F + (long)k * hx * ldj;
-        const wf_real inv_scale = WR(1.0) / ((wf_real)nx * (wf_real)ny);
-        const int Nx = c.Nx;
-        wfc *tw = smem, *bufa = smem + nx, *bufb = bufa + pairs * nx;
-        for (int t = threadIdx.x; t < nx; t += blockDim.x) {
-            wf_real2 w = sp.twx[t];
-            tw[t].re = w.x;
-            tw[t].im = -w.y;
-        }
-        if (threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
-        for (int t = threadIdx.x; t < pairs * nx; t += blockDim.x) {
-            const int s = t % pairs, r = t / pairs;
-            const int ja = j0 + 2 * s, jb = ja + 1;
-            wfc A = {WR(0.0), WR(0.0)}, B = {WR(0.0), WR(0.0)};
-            const int conj = r >= hx;
-            const int rr = conj ? nx - r : r;
-            if (ja < ny) {
-                wf_real2 x = src[(long)rr * ldj + ja];
-                A.re = x.x;
-                A.im = x.y;
-                if (jb < ny) {
-                    wf_real2 y = src[(long)rr * ldj + jb];
-                    B.re = y.x;
-                    B.im = y.y;
-                }
-            }
-            bufa[s * nx + r] = wf_pack_pair(A, B, conj);
-        }
-        __syncthreads();
-        wfc *res = wf_lds_fft(bufa, bufb, nx, pairs, rad, tw);
-        for (int t = threadIdx.x; t < pairs * (Nx - 1); t += blockDim.x) {
-            const int s = t / (Nx - 1), i = t - s * (Nx - 1);
-            const int ja = j0 + 2 * s, jb = ja + 1;
-            if (ja >= ny) continue;
-            wf_put_p(c, p, i, ja, k, res[s * nx + i].re * inv_scale, dmax, pabs);
-            if (jb < ny) wf_put_p(c, p, i, jb, k, res[s * nx + i].im * inv_scale, dmax, pabs);
-        }
-    }
+    if (NX <= 0 && threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
+    wf_inv_fx_rows<NX>(c, sp, p, smem, rad, g, k, dmax, pabs);
     wf_block_max_store(dmax, &sp.pmax[blockIdx.x]);
     if constexpr (WF_MIXED) {
         __syncthreads();
@@ -897,9 +799,6 @@ __global__ __launch_bounds__(WF_NT) void k_iter_check_batch(const WfPressItem *_
 
 /* ------------------------------------------------------------- launchers ---- */
 
-/* lengths with a compile-time Stockham plan (x-transforms) */
-static bool wf_planned(int n) { return n == 63 || n == 127 || n == 255 || n == 511; }
-
 /* dynamic LDS of an x-transform kernel: twiddles + one buffer (compile-time
  * plan, in place) or two buffers (run-time radices) */
 static size_t wf_fx_lds(int n, int nseq) {
@@ -922,7 +821,12 @@ static size_t wf_fy_lds(int n, int nseq) {
             case 127: hipLaunchKernelGGL(KERNEL<127>, grd, blk, lds, s, __VA_ARGS__); break;            \
             case 255: hipLaunchKernelGGL(KERNEL<255>, grd, blk, lds, s, __VA_ARGS__); break;            \
             case 511: hipLaunchKernelGGL(KERNEL<511>, grd, blk, lds, s, __VA_ARGS__); break;            \
-            default: hipLaunchKernelGGL(KERNEL<0>, grd, blk, lds, s, __VA_ARGS__); break;               \
+            default:                                                                                    \
+                if (n <= WF_NX_SHORT)                                                                   \
+                    hipLaunchKernelGGL(KERNEL<0>, grd, blk, lds, s, __VA_ARGS__);                       \
+                else                                                                                    \
+                    hipLaunchKernelGGL(KERNEL<-1>, grd, blk, lds, s, __VA_ARGS__);                      \
+                break;                                                                                  \
         }                                                                                               \
     } while (0)
 
@@ -944,7 +848,12 @@ static size_t wf_fy_lds(int n, int nseq) {
             case 127: hipLaunchKernelGGL((KERNEL<127, MODE>), grd, blk, lds, s, __VA_ARGS__); break;    \
             case 255: hipLaunchKernelGGL((KERNEL<255, MODE>), grd, blk, lds, s, __VA_ARGS__); break;    \
             case 511: hipLaunchKernelGGL((KERNEL<511, MODE>), grd, blk, lds, s, __VA_ARGS__); break;    \
-            default: hipLaunchKernelGGL((KERNEL<0, MODE>), grd, blk, lds, s, __VA_ARGS__); break;       \
+            default:                                                                                    \
+                if (n <= WF_NX_SHORT)                                                                   \
+                    hipLaunchKernelGGL((KERNEL<0, MODE>), grd, blk, lds, s, __VA_ARGS__);               \
+                else                                                                                    \
+                    hipLaunchKernelGGL((KERNEL<-1, MODE>), grd, blk, lds, s, __VA_ARGS__);              \
+                break;                                                                                  \
         }                                                                                               \
     } while (0)
 
