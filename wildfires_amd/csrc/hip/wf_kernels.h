@@ -139,6 +139,12 @@ struct WfIterCtl {
     int solves; /* solves performed */
     double err; /* last max |p_new - p_old| */
 };
+/* Its copy in mapped host memory, written by every check (done last): the
+ * host follows the iteration by it and takes the results from it. */
+struct WfHostFlag {
+    int done, solves, iters;
+    double err;
+};
 
 /* Row pairs per workgroup in the x-transforms and kx columns per workgroup in
  * the y-transform, for a transform length n. */
@@ -199,7 +205,7 @@ struct WfSpectral {
     const wf_real *beta;           /* nz: 2/(dz_{k-1} dz_k) for 1 <= k <= nz-2 */
     const wf_real *rho;            /* rho^n on every node (variable density) */
     WfIterCtl *ctl;
-    int *hflag;                    /* mapped host memory: [0] done, [1] solves finished */
+    WfHostFlag *hflag;             /* mapped host memory */
     /* coefficient-plane form (wf_planes.hip, FP64), used when pl is set */
     int pl;
     int pl_ld;          /* row stride of a plane: ny rounded up to 16 */

@@ -189,20 +189,19 @@ __device__ __forceinline__ void wf_iter_check_body(const WfSpectral &sp, double 
 #if WF_MIXED
     tol_eff = (rtol * pabs > tol_eff) ? rtol * pabs : tol_eff;
 #endif
+    const int met = err <= tol_eff;
+    const int iters = met ? m : m + 1, done = met || m + 1 >= max_iter;
     ctl->err = err;
     ctl->solves = m + 1;
-    int done;
-    if (err <= tol_eff) {
-        done = 1;
-        ctl->iters = m;
-    } else {
-        ctl->iters = m + 1;
-        done = (m + 1 >= max_iter) ? 1 : 0;
-    }
+    ctl->iters = iters;
     ctl->done = done;
-    volatile int *hf = sp.hflag;
-    hf[1] = m + 1;
-    hf[0] = done;
+    volatile WfHostFlag *hf = sp.hflag;
+    hf->err = err;
+    hf->iters = iters;
+    hf->solves = m + 1;
+    if (!done) return;
+    __threadfence_system();
+    hf->done = 1;
     __threadfence_system();
 }
 /* Block index of a first pass whose block 0 checks the previous solve

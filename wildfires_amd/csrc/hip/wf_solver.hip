@@ -77,8 +77,8 @@ struct Solver {
     wf_real *Tsrc, *rho;
     int have_Tsrc;
     WfIterCtl *ctl;
-    int *hflag;      /* mapped pinned host memory: [0] done, [1] solves finished */
-    int *hflag_dev;  /* its device address */
+    WfHostFlag *hflag;     /* mapped pinned host memory */
+    WfHostFlag *hflag_dev; /* its device address */
     int method; /* 0 Euler, 1 RK2, 2 RK4 */
     int stage_split; /* 1: derived pass + stage pass also without the closure (WF_STAGE_FORM=split) */
     int stage_shape; /* stage tile shape (-1 until tuned at the first stage) */
@@ -283,10 +283,9 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     WF_HIP(hipMalloc((void **)&s->rho, sizeof(wf_real) * s->N));
     WF_HIP(hipMalloc((void **)&s->ctl, sizeof(WfIterCtl)));
     WF_HIP(hipMemset(s->ctl, 0, sizeof(WfIterCtl)));
-    WF_HIP(hipHostMalloc((void **)&s->hflag, 2 * sizeof(int), hipHostMallocMapped));
+    WF_HIP(hipHostMalloc((void **)&s->hflag, sizeof(WfHostFlag), hipHostMallocMapped));
     WF_HIP(hipHostGetDevicePointer((void **)&s->hflag_dev, s->hflag, 0));
-    s->hflag[0] = 0;
-    s->hflag[1] = 0;
+    memset(s->hflag, 0, sizeof(WfHostFlag));
 
     /* grid tables evaluated on the host exactly as the reference evaluates them */
     const double *z = P->z;
@@ -781,12 +780,18 @@ static int wf_integrate(Solver *s) {
 }
 
 /* Pressure solve of src/cu/pressure.cu:506-606 for y* = Ys, y_n = Yn.  The
- * solves are queued without host synchronisation; k_iter_check tests
- * convergence on the device after each solve, turns the remaining kernels
- * into no-ops and writes the flag and the solve count to mapped host memory.  The
- * host keeps at most WF_LOOKAHEAD solves queued ahead of the device and stops
- * queueing once the flag is set. */
-#define WF_LOOKAHEAD 6
+ * solves are queued without host synchronisation; the check of each (done
+ * beside the next one's first pass) tests convergence on the device, turns the
+ * remaining kernels into no-ops and writes the flag, the solve count and the
+ * error to mapped host memory.  The host keeps at most WF_LOOKAHEAD solves
+ * queued ahead of the checked ones, stops queueing once the flag is set, takes
+ * the results from it and goes on queueing the step behind the no-ops.
+ * Three: the one that runs, the next, and one more for the lag of the count
+ * (a solve is counted by the first pass of the next).  64x64x32 mixed, one
+ * step: 424 us with six ahead, a copy of the results and a wait for the stream
+ * behind them; 397 with six and the results in the flag; 378 with three (379
+ * with two, which in FP64 starves the device: 845 us against 825). */
+#define WF_LOOKAHEAD 3
 static int wf_max_iter(const Parameters &P) { return (P.variable_density == 0) ? 1 : P.pressure_solver_iter; }
 
 /* control reset and rho^n of a solve (launches only: capturable) */
@@ -839,39 +844,44 @@ static int wf_pressure_rest(Solver *s, const WfState &ys, const WfState &yn, int
         s->last_iters = 0;
         return WF_OK;
     }
-    volatile int *hf = s->hflag;
-    int rc;
-    for (int m = m0; m < max_iter; m++) {
-        if (m > 0 && hf[0]) break;
+    volatile WfHostFlag *hf = s->hflag;
+    int rc, m = m0;
+    /* the stream's state while the flag is not set */
+    const auto drained = [&](bool *empty) -> int {
+        for (int spin = 0; spin < 64 && !hf->done; spin++) __builtin_ia32_pause();
+        const hipError_t e = hipStreamQuery(s->stream);
+        *empty = e == hipSuccess;
+        if (e != hipSuccess && e != hipErrorNotReady) return wf_fail(WF_E_DEVICE, "pressure solve: %s", hipGetErrorString(e));
+        return WF_OK;
+    };
+    while (m < max_iter && !(m > 0 && hf->done)) {
         /* the solves before m0 have been checked */
         if ((rc = wf_pressure_one(s, ys, yn, m, max_iter, m > m0, m + 1 >= max_iter))) return rc;
-        if (m + 1 >= max_iter) break;
-        /* wait until the device is within WF_LOOKAHEAD solves (the count
-         * lags a solve: solve m is counted by solve m + 1's first pass); if
-         * the stream drains without the flag advancing, fall through and keep
-         * queueing */
-        while (!hf[0] && (m + 1) - hf[1] >= WF_LOOKAHEAD) {
-            if (hipStreamQuery(s->stream) == hipSuccess) break;
-        }
+        m++;
+        /* wait until the device is within WF_LOOKAHEAD solves; if the stream
+         * drains without the count advancing, keep queueing */
+        bool empty = false;
+        while (m < max_iter && !empty && !hf->done && m - hf->solves >= WF_LOOKAHEAD)
+            if ((rc = drained(&empty))) return rc;
     }
-    WfIterCtl ctl;
-    WF_HIP(hipMemcpyAsync(&ctl, s->ctl, sizeof(ctl), hipMemcpyDeviceToHost, s->stream));
-    WF_HIP(hipStreamSynchronize(s->stream));
-    s->press_solves += ctl.solves;
+    for (bool empty = false; !hf->done;) {
+        if (empty) return wf_fail(WF_E_DEVICE, "pressure solve: the iteration ended without its result");
+        if ((rc = drained(&empty))) return rc;
+    }
+    s->press_solves += hf->solves;
     if (s->P.variable_density == 0) {
         s->last_err = 0.0;
         s->last_iters = 0;
     } else {
-        s->last_err = ctl.err;
-        s->last_iters = ctl.iters;
+        s->last_err = hf->err;
+        s->last_iters = hf->iters;
     }
     return WF_OK;
 }
 
 static int wf_pressure_solve(Solver *s, char *Ys_buf, char *Yn_buf) {
     const WfState ys = wf_view(s, Ys_buf), yn = wf_view(s, Yn_buf);
-    s->hflag[0] = 0;
-    s->hflag[1] = 0;
+    memset(s->hflag, 0, sizeof(WfHostFlag));
     int rc = wf_pressure_begin(s, yn);
     if (rc) return rc;
     return wf_pressure_rest(s, ys, yn, 0);
@@ -1648,8 +1658,7 @@ int ens_step(Ensemble *e, int step0, int n_steps) {
     for (int n = step0; n < step0 + n_steps; n++) {
         const int par = e->parity;
         for (int i = 0; i < e->n; i++) {
-            e->m[i]->hflag[0] = 0;
-            e->m[i]->hflag[1] = 0;
+            memset(e->m[i]->hflag, 0, sizeof(WfHostFlag));
         }
         if (e->use_graph) {
             if (!e->exec[par]) {
@@ -1678,7 +1687,7 @@ int ens_step(Ensemble *e, int step0, int n_steps) {
             s->stream = (K > 1) ? e->side[i % K] : e->stream;
             const WfState ys = wf_view(s, s->state[2]), yn = wf_view(s, s->state[s->i_yn]);
             const int max_iter = wf_max_iter(s->P);
-            if (max_iter > 0 && !s->hflag[0] && e->budget < max_iter) {
+            if (max_iter > 0 && !s->hflag->done && e->budget < max_iter) {
                 /* not converged within the budget: the further solves of its solo run */
                 if ((rc = wf_pressure_rest(s, ys, yn, e->budget))) break;
             } else if (max_iter > 0) {
