@@ -149,3 +149,13 @@ def test_mixed_run_time_lengths_close_to_fp64(tmp_path, monkeypatch, nx, ny, nz)
     print("%dx%dx%d mixed vs fp64 %.3e" % (nx, ny, nz, rel_l2(pm, pd)), flush=True)
     assert rel_l2(pm, pd) <= 2e-5
     assert im == idd
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(6, 34, 9), (8, 65, 10), (12, 66, 17), (5, 98, 18), (14, 130, 33), (8, 40, 129),
+                                      (8, 70, 130)])
+def test_mixed_tridiagonal_tiles_close_to_fp64(tmp_path, monkeypatch, nx, ny, nz):
+    """Tridiagonal solve of the mixed form: 33 to 129 systems in ky (tiles of
+    64 whose FP64 halves hold 32, 1, 2, 33 and 64), fewer kx columns than the
+    FP64 ones, levels at the edges of the chunks of 8 and 16.  The bound of the
+    run-time lengths."""
+    test_mixed_run_time_lengths_close_to_fp64(tmp_path, monkeypatch, nx, ny, nz)

@@ -33,6 +33,9 @@ namespace WF_NS {
 /* Row pairs of an x-transform workgroup compiled for length NX, and the most
  * elements a thread of it takes.  NX = 0 and -1 are the run-time lengths up
  * to 300 and above. */
+/* FP32 chunks of 8 levels: 8 waves per SIMD, so that two 16-wave workgroups
+ * share a CU (256x256x128: 512 workgroups, one round of them) */
+#define WF_THOMAS_ATTR(LC) __attribute__((amdgpu_waves_per_eu((WF_MIXED && (LC) == 8) ? 8 : 4)))
 #define WF_NX_SHORT 300
 template <int NX>
 struct WfFx {
@@ -284,146 +287,169 @@ __global__ void k_pivots(WfSpectral sp, double *UB) {
  * in place in F (src/cu/pressure.cu:418-443 with the right-hand side of
  * 473-504):  y_0 = d_0, y_k = d_k - L_k y_{k-1};  x_{nz-1} = y_{nz-1}/u_{nz-1},
  * x_k = (y_k - c_k x_{k+1})/u_k, in arithmetic type TA.
- * Wave w owns levels [w LC, w LC + LC) of all 64 systems and keeps them in
+ * Wave w owns levels [w LC, w LC + LC) of its systems and keeps them in
  * registers.  Both recurrences are affine in the value entering the chunk, so
  * each wave runs them from a zero entry value while carrying the coefficient
  * of the entry value (products of -L_k, resp. of -c_k/u_k); the waves then
- * combine their chunk ends through LDS in order and add the correction. */
-template <int LC, typename TA>
-__device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, wf_cx<TA> (*sv)[64], TA (*sg)[64]) {
+ * combine their chunk ends through LDS in order and add the correction.
+ * A lane holds NC components of its system (ky j of kx r): both (64 systems
+ * to a wave), or component comp alone (32 systems).  All loads go out first and
+ * no level has a branch of its own: the levels above the top read the top's
+ * entries, and the tables (padded to whole chunks: a = c = 0, beta = 1) keep
+ * their values finite and apart from the others. */
+template <typename TA, int NC>
+struct WfThomasLds {
+    TA v[WF_THOMAS_MAX_CHUNKS][64][NC], g[WF_THOMAS_MAX_CHUNKS][64];
+};
+template <int LC, typename TA, int NC>
+__device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLds<TA, NC> &L, int j, int r,
+                                                int comp) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int C = blockDim.x >> 6;
-    const int j = blockIdx.x * 64 + lane, r = blockIdx.y;
     const int nz = sp.nz;
     const bool ok = j < sp.ny;
     const long slab = (long)sp.hx * sp.ldj;
-    const long o = (long)r * sp.ldj + (ok ? j : 0);
+    const long row = (long)r * sp.ldj; /* uniform: a level's entries are at a scalar base + at */
+    const unsigned jj = ok ? j : 0, at = 2 * jj + comp;
     const int k0 = w * LC;
-    const TA K2 = ok ? wf_tab<TA>(sp.kx2, sp.kx2d, r) + wf_tab<TA>(sp.ky2, sp.ky2d, j) : (TA)0.0;
-    const TA c0 = (TA)sp.c0a - (TA)0.5 * (TA)sp.dz0 * K2 - (TA)sp.c0b;
-    wf_cx<TA> y[LC];
-    TA g[LC], ru[LC];
-    TA u = (w > 0 && ok) ? (TA)sp.UB[o + w * slab] : (TA)sp.b0; /* pivot entering the chunk */
+    TA y[LC][NC], g[LC], ru[LC], pt[NC];
 #pragma unroll
     for (int t = 0; t < LC; t++) {
-        const int k = k0 + t;
-        y[t] = wf_cx<TA>{(TA)0.0, (TA)0.0};
-        g[t] = (TA)0.0;
-        ru[t] = (TA)0.0;
-        if (ok && k < nz) {
-            if (k == 0) {
-                const wf_cx<TA> f1 = wf_ldF<TA>(sp.F, o + slab);
-                y[t] = wf_cx<TA>{(TA)0.5 * (TA)sp.dz0 * f1.x, (TA)0.5 * (TA)sp.dz0 * f1.y};
-                u = (TA)sp.b0;
-            } else {
-                wf_cx<TA> d = wf_ldF<TA>(sp.F, o + k * slab);
-                if (k == nz - 1) {
-                    const wf_cx<TA> pt = wf_ldF<TA>(sp.Ptop, o);
-                    d.x = d.x - pt.x / (TA)sp.top_div;
-                    d.y = d.y - pt.y / (TA)sp.top_div;
-                }
-                y[t] = d;
-                TA l;
-                u = wf_pivot_next<TA>(sp, u, k, K2, c0, &l);
-                g[t] = l;
-            }
-            ru[t] = (TA)1.0 / u;
+        int k = min(k0 + t, nz - 1);
+        if (t == 0) k = max(k, 1); /* level 0 takes level 1's right-hand side */
+#pragma unroll
+        for (int q = 0; q < NC; q++) y[t][q] = (TA)((const wf_real *)(sp.F + row + k * slab))[at + q];
+    }
+#pragma unroll
+    for (int q = 0; q < NC; q++)
+        pt[q] = (k0 + LC >= nz) ? (TA)((const wf_real *)(sp.Ptop + row))[at + q] / (TA)sp.top_div : (TA)0.0;
+    TA u = w ? (TA)(sp.UB + row + w * slab)[jj] : (TA)sp.b0; /* pivot entering the chunk */
+    const TA K2 = wf_tab<TA>(sp.kx2, sp.kx2d, r) + wf_tab<TA>(sp.ky2, sp.ky2d, jj);
+    const TA half_dz0 = (TA)0.5 * (TA)sp.dz0;
+    const TA c0 = (TA)sp.c0a - half_dz0 * K2 - (TA)sp.c0b;
+    const TA ck0 = w ? wf_tab<TA>(sp.tc, sp.tcd, k0) : c0; /* c_{k0} */
+    /* the pivots u_k (wf_pivot_next's operations), L_k and 1/u_k */
+#pragma unroll
+    for (int t = 0; t < LC; t++) {
+        const int km = (t > 0) ? k0 + t - 1 : max(k0 - 1, 0);
+        const TA bk = -(K2 + wf_tab<TA>(sp.beta, sp.betad, k0 + t));
+        const TA l = wf_tab<TA>(sp.ta, sp.tad, km) / u;
+        u = bk - l * ((t == 1) ? ck0 : wf_tab<TA>(sp.tc, sp.tcd, km));
+        g[t] = l;
+        if (t == 0) {
+            u = w ? u : (TA)sp.b0;
+            g[0] = w ? l : (TA)0.0;
         }
+        ru[t] = (TA)1.0 / u;
     }
     /* forward elimination, entry value 0, coefficient G of the entry value */
-    wf_cx<TA> acc = {(TA)0.0, (TA)0.0};
-    TA G = (TA)1.0;
+    TA acc[NC], G = (TA)1.0;
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+        acc[q] = (TA)0.0;
+        y[0][q] = w ? y[0][q] : half_dz0 * y[0][q];
+    }
 #pragma unroll
     for (int t = 0; t < LC; t++) {
-        const int k = k0 + t;
-        if (k == 0) {
-            acc = y[0];
-            G = (TA)0.0;
-        } else {
-            const TA m = g[t];
-            acc.x = y[t].x - m * acc.x;
-            acc.y = y[t].y - m * acc.y;
-            G = -m * G;
-            y[t] = acc;
+        const TA m = g[t];
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            const TA d = y[t][q] - ((k0 + t == nz - 1) ? pt[q] : (TA)0.0);
+            y[t][q] = acc[q] = d - m * acc[q];
         }
-        g[t] = G;
-    }
-    sv[w][lane] = acc;
-    sg[w][lane] = G;
-    __syncthreads();
-    wf_cx<TA> Y = {(TA)0.0, (TA)0.0};
-    for (int q = 0; q < w; q++) {
-        const wf_cx<TA> e = sv[q][lane];
-        const TA gq = sg[q][lane];
-        Y.x = e.x + gq * Y.x;
-        Y.y = e.y + gq * Y.y;
+        g[t] = G = -m * G;
     }
 #pragma unroll
-    for (int t = 0; t < LC; t++) {
-        y[t].x = y[t].x + g[t] * Y.x;
-        y[t].y = y[t].y + g[t] * Y.y;
+    for (int q = 0; q < NC; q++) L.v[w][lane][q] = acc[q];
+    L.g[w][lane] = G;
+    __syncthreads();
+    TA Y[NC];
+#pragma unroll
+    for (int q = 0; q < NC; q++) Y[q] = (TA)0.0;
+#pragma unroll 4
+    for (int s = 0; s < w; s++) {
+        const TA gs = L.g[s][lane];
+#pragma unroll
+        for (int q = 0; q < NC; q++) Y[q] = L.v[s][lane][q] + gs * Y[q];
     }
+#pragma unroll
+    for (int t = 0; t < LC; t++)
+#pragma unroll
+        for (int q = 0; q < NC; q++) y[t][q] = y[t][q] + g[t] * Y[q];
     __syncthreads();
     /* back substitution, entry value x_{k0+LC} = 0, coefficient H */
-    wf_cx<TA> xa = {(TA)0.0, (TA)0.0};
-    TA H = (TA)1.0;
+    TA xa[NC], H = (TA)1.0;
+#pragma unroll
+    for (int q = 0; q < NC; q++) xa[q] = (TA)0.0;
 #pragma unroll
     for (int t = LC - 1; t >= 0; t--) {
-        const int k = k0 + t;
-        if (k >= nz) continue;
-        if (k == nz - 1) {
-            xa.x = y[t].x * ru[t];
-            xa.y = y[t].y * ru[t];
-            H = (TA)0.0;
-        } else {
-            const TA ck = (k == 0) ? c0 : wf_tab<TA>(sp.tc, sp.tcd, k);
-            xa.x = (y[t].x - ck * xa.x) * ru[t];
-            xa.y = (y[t].y - ck * xa.y) * ru[t];
-            H = (-ck * ru[t]) * H;
-        }
-        y[t] = xa;
-        g[t] = H;
+        const TA ck = (t == 0) ? ck0 : wf_tab<TA>(sp.tc, sp.tcd, k0 + t); /* 0 at the top and above */
+#pragma unroll
+        for (int q = 0; q < NC; q++) y[t][q] = xa[q] = (y[t][q] - ck * xa[q]) * ru[t];
+        g[t] = H = (-ck * ru[t]) * H;
     }
-    sv[w][lane] = xa;
-    sg[w][lane] = H;
+#pragma unroll
+    for (int q = 0; q < NC; q++) L.v[w][lane][q] = xa[q];
+    L.g[w][lane] = H;
     __syncthreads();
-    wf_cx<TA> X = {(TA)0.0, (TA)0.0};
-    for (int q = C - 1; q > w; q--) {
-        const wf_cx<TA> e = sv[q][lane];
-        const TA hq = sg[q][lane];
-        X.x = e.x + hq * X.x;
-        X.y = e.y + hq * X.y;
+    TA X[NC];
+#pragma unroll
+    for (int q = 0; q < NC; q++) X[q] = (TA)0.0;
+#pragma unroll 4
+    for (int s = C - 1; s > w; s--) {
+        const TA hs = L.g[s][lane];
+#pragma unroll
+        for (int q = 0; q < NC; q++) X[q] = L.v[s][lane][q] + hs * X[q];
     }
     if (!ok) return;
 #pragma unroll
     for (int t = 0; t < LC; t++) {
         const int k = k0 + t;
-        if (k < nz) sp.F[o + k * slab] = wf_make2((wf_real)(y[t].x + g[t] * X.x), (wf_real)(y[t].y + g[t] * X.y));
+        if (k >= nz) break;
+#pragma unroll
+        for (int q = 0; q < NC; q++)
+            ((wf_real *)(sp.F + row + k * slab))[at + q] = (wf_real)(y[t][q] + g[t] * X[q]);
     }
 }
 
 template <int LC>
 __device__ __forceinline__ void wf_thomas_body(const WfSpectral &sp) {
     if (sp.ctl->done) return;
-    __shared__ wf_cx<double> sv[WF_THOMAS_MAX_CHUNKS][64];
-    __shared__ double sg[WF_THOMAS_MAX_CHUNKS][64];
+    const int lane = threadIdx.x & 63, jlo = blockIdx.x * 64;
 #if WF_MIXED
-    /* a workgroup holding one of the lowest wavenumbers (kx index below
-     * low_kx, ky index within low_ky of 0 or of ny) solves in FP64: those
-     * systems are singular or nearly so under the Neumann z conditions */
-    const int jlo = blockIdx.x * 64, jhi = (jlo + 63 < sp.ny - 1) ? jlo + 63 : sp.ny - 1;
-    const bool low = ((int)blockIdx.y < sp.low_kx) && (jlo < sp.low_ky || sp.ny - jhi < sp.low_ky);
+    /* a tile of 64 systems holding one of the lowest wavenumbers (kx index
+     * below low_kx, ky index within low_ky of 0 or of ny) is solved in FP64:
+     * those systems are singular or nearly so under the Neumann z conditions.
+     * Two workgroups share such a tile, a component of a system to a lane: its
+     * FP64 values then fit the registers of an FP32 workgroup's (64, so that
+     * two of 16 waves share a CU), and its chain of FP64 divisions and
+     * combines, the longest of the launch, has half the work.  The second
+     * halves are low_kx rows of workgroups before the kx columns'.  us, with
+     * a complex FP64 system to a lane, 105 registers and a branch per level
+     * before: 64x64x32 8.6 -> 5.3, 128x128x64 10.8 -> 8.2, 201x151x81 16 ->
+     * 13.8, 256x256x128 23.2 -> 20.5 (16.2 without the FP64 systems, whose
+     * extra workgroups there start when the first others end).  Both halves
+     * by one workgroup in turn: 9.5, 16.1, 20.7, 29.4. */
+    __shared__ union {
+        WfThomasLds<float, 2> f;
+        WfThomasLds<double, 1> d;
+    } L;
+    const int second = (int)blockIdx.y < sp.low_kx;
+    const int r = second ? (int)blockIdx.y : (int)blockIdx.y - sp.low_kx;
+    const int jhi = (jlo + 63 < sp.ny - 1) ? jlo + 63 : sp.ny - 1;
+    const bool low = r < sp.low_kx && (jlo < sp.low_ky || sp.ny - jhi < sp.low_ky);
     if (low)
-        wf_thomas_solve<LC, double>(sp, sv, sg);
-    else
-        wf_thomas_solve<LC, float>(sp, (wf_cx<float>(*)[64])sv, (float(*)[64])sg);
+        wf_thomas_solve<LC, double, 1>(sp, L.d, jlo + 32 * second + (lane >> 1), r, lane & 1);
+    else if (!second)
+        wf_thomas_solve<LC, float, 2>(sp, L.f, jlo + lane, r, 0);
 #else
-    wf_thomas_solve<LC, double>(sp, sv, sg);
+    __shared__ WfThomasLds<double, 2> L;
+    wf_thomas_solve<LC, double, 2>(sp, L, jlo + lane, (int)blockIdx.y, 0);
 #endif
 }
 template <int LC>
-__global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) void k_thomas(WfSpectral sp) {
+__global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) WF_THOMAS_ATTR(LC) void k_thomas(WfSpectral sp) {
     wf_thomas_body<LC>(sp);
 }
 
@@ -772,7 +798,7 @@ __global__ __launch_bounds__(WF_NT) void k_fy_batch(const WfPressItem *__restric
 }
 
 template <int LC>
-__global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) void k_thomas_batch(const WfPressItem *__restrict__ tab) {
+__global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) WF_THOMAS_ATTR(LC) void k_thomas_batch(const WfPressItem *__restrict__ tab) {
     const WfPressItem it = wf_press_load(tab);
     wf_thomas_body<LC>(it.sp);
 }
@@ -908,8 +934,8 @@ hipError_t wf_launch_pivots(const WfSpectral &sp, double *UB, hipStream_t s) {
 }
 
 hipError_t wf_launch_thomas(const WfSpectral &sp, hipStream_t s) {
-    dim3 grd((sp.ny + 63) / 64, sp.hx, 1);
     const int chunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
+    dim3 grd((sp.ny + 63) / 64, sp.hx + sp.low_kx, 1);
     if (sp.thomas_lc == 4) {
 #if WF_MIXED
         return hipErrorInvalidValue;
@@ -981,8 +1007,8 @@ hipError_t wf_launch_fy_batch(const WfSpectral &sp, const WfPressItem *tab, int 
 }
 
 hipError_t wf_launch_thomas_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s) {
-    dim3 grd((sp.ny + 63) / 64, sp.hx, nm);
     const int chunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
+    dim3 grd((sp.ny + 63) / 64, sp.hx + sp.low_kx, nm);
     if (sp.thomas_lc == 4) {
 #if WF_MIXED
         return hipErrorInvalidValue;

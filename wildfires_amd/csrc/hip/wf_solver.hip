@@ -461,7 +461,9 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
     for (int q = 0; q < sp.ny; q++) ky2[q] = P->ky[q] * P->ky[q];
     if ((rc = wf_upload_real(&s->kx2, kx2.data(), sp.hx))) return rc;
     if ((rc = wf_upload_real(&s->ky2, ky2.data(), sp.ny))) return rc;
-    std::vector<double> ta(sp.nz, 0.0), tc((sp.nz + 15) & ~15, 0.0), beta(sp.nz, 0.0);
+    /* padded to the longest chunk of k_thomas, whose rows above the top are x = y / u */
+    const size_t npad = (sp.nz + 15) & ~15;
+    std::vector<double> ta(npad, 0.0), tc(npad, 0.0), beta(npad, 1.0);
     for (int k = 0; k < Nz - 2; k++) {
         double dz_k = z[k + 1] - z[k], dz_kp1 = z[k + 2] - z[k + 1];
         ta[k] = 2 / (dz_k * (dz_k + dz_kp1));
@@ -471,19 +473,20 @@ static int wf_create_impl(Solver *s, const Parameters *P) {
             beta[k] = 2 / (dz_km1 * dz_k);
         }
     }
-    if ((rc = wf_upload_real(&s->ta, ta.data(), sp.nz))) return rc;
+    beta[Nz - 2] = 2 / ((z[Nz - 2] - z[Nz - 3]) * (z[Nz - 1] - z[Nz - 2])); /* beta_top */
+    if ((rc = wf_upload_real(&s->ta, ta.data(), npad))) return rc;
     if ((rc = wf_upload_real(&s->tc, tc.data(), tc.size()))) return rc;
-    if ((rc = wf_upload_real(&s->beta, beta.data(), sp.nz))) return rc;
+    if ((rc = wf_upload_real(&s->beta, beta.data(), npad))) return rc;
 #if WF_MIXED
     if ((rc = wf_upload(&s->kx2d, kx2.data(), sp.hx))) return rc;
     if ((rc = wf_upload(&s->ky2d, ky2.data(), sp.ny))) return rc;
-    if ((rc = wf_upload(&s->tad, ta.data(), sp.nz))) return rc;
+    if ((rc = wf_upload(&s->tad, ta.data(), npad))) return rc;
     if ((rc = wf_upload(&s->tcd, tc.data(), tc.size()))) return rc;
-    if ((rc = wf_upload(&s->betad, beta.data(), sp.nz))) return rc;
+    if ((rc = wf_upload(&s->betad, beta.data(), npad))) return rc;
     /* the systems solved in FP64: kx index < low_kx and ky index within
      * low_ky of 0 or ny (WF_MIXED_LOW_KX / WF_MIXED_LOW_KY override 4, 4) */
     const char *ekx = getenv("WF_MIXED_LOW_KX"), *eky = getenv("WF_MIXED_LOW_KY");
-    sp.low_kx = ekx ? atoi(ekx) : 4;
+    sp.low_kx = std::max(0, std::min(ekx ? atoi(ekx) : 4, sp.hx));
     sp.low_ky = eky ? atoi(eky) : 4;
 #else
     sp.low_kx = 0;
