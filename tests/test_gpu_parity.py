@@ -356,3 +356,30 @@ def test_deepest_grid_matches_oracle(tmp_path, monkeypatch):
     assert gs == os_
     for name, e in errs.items():
         assert e <= 1e-10, (name, e)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nx,ny,nz", [(256, 260, 7), (256, 258, 6), (256, 257, 8), (64, 258, 7), (64, 64, 9), (512, 6, 6),
+                                      (128, 520, 6), (256, 516, 6)])
+def test_compile_time_x_lengths(tmp_path, monkeypatch, precision, nx, ny, nz):
+    """x-transforms of the compile-time lengths by their row maps: whole
+    wavefronts of one row pair, the last column's and the last rows' periodic
+    neighbours, the last group of 4 or 8 row pairs holding one to all of them
+    (the last with a single row or not), against the oracle: four solves of
+    the iteration within 1e-11 in FP64 and, as the mixed form's other length
+    tests, within 2e-5 in FP32."""
+    from oracle import oracle
+    from wildfires_amd import api
+    prm = make_params(tmp_path, "small_flat", Nx=nx, Ny=ny, Nz=nz, x_max=2.0 * (nx - 1), y_max=2.0 * (ny - 1),
+                      z_max=0.5 * (nz - 1), pressure_solver_iter=4)
+    y, p = perturbed_state(prm)
+    O = oracle.Oracle(prm.ptr)
+    y1 = y + prm.p.dt * O.phi(y)
+    monkeypatch.setenv("WF_MIXED_PRESSURE_RTOL", "0")
+    with api.Solver(prm, precision) as solver:
+        pg, _, ig = solver.pressure(y1, y, p)
+    po = p.copy()
+    _, io, _ = O.pressure(y1, y, po)
+    print("%dx%dx%d %s rel %.2e" % (nx, ny, nz, precision, rel_l2(pg, po)), flush=True)
+    assert rel_l2(pg, po) <= (1e-11 if precision == "fp64" else 2e-5)
+    assert ig == io

@@ -531,6 +531,74 @@ __device__ __forceinline__ void wf_f2_phase_b(const wfc *buf, const wf_real2 *tw
     for (int n1 = 0; n1 < N1; n1++) y[n1] = col[n1];
     wf_dft_reg<N1, N2, SIGN>(y, tw, out);
 }
+
+/* ------------------------------------------------------------------------
+ * Register form of the compile-time Stockham plan with three odd radices
+ * R1 R2 R3 (255 = 3 5 17), for the FP32 x-transforms.  The stages compute what
+ * wf_stage_ip computes, term for term and bit for bit (a twiddle's products
+ * are spelled out in the form its compiled contraction takes, the sums of a
+ * DFT are the same chains), but the values between the first two stay in
+ * registers, each value crosses LDS once, not three times, with two barriers
+ * instead of six, and the DFT constants come by scalar loads, not from LDS
+ * one by one: 7.2 M vector instructions instead of 16 M in P5 at 256x256x128,
+ * whose time, bound by them before and by its two phases' latency now, goes
+ * from 30.4 to 25.5 us; P1 stays at 32.7 (its loads).  With 4 row pairs to a
+ * workgroup instead of 8, 32.6 and 33.2.  In FP64 its registers (145-198)
+ * leave too few waves: P5 47 us against 44 in place, P1 84 against 76.
+ * Input of block g of the last radix: x[g + R3 m], m < R1 R2.
+ * Phase A: one thread per (sequence, g) runs the radices R1 and R2 on its
+ * R1 R2 inputs and twiddles the outputs for the last radix.
+ * Phase B: one thread per (sequence, j), j < R1 R2, runs the radix R3.
+ * ---------------------------------------------------------------------- */
+__host__ __device__ constexpr int wf_rx_a(int n) { return (WF_MIXED && n == 255) ? 15 : 0; }
+__host__ __device__ constexpr int wf_rx_b(int n) { return (WF_MIXED && n == 255) ? 17 : 0; }
+
+/* a w, or a conj(w) for the inverse transform */
+template <int SIGN>
+__device__ __forceinline__ wfc wf_twiddle(wfc a, wf_real2 w) {
+    const wf_real wi = (SIGN < 0) ? w.y : -w.y;
+    wfc r;
+    r.re = wf_fma(a.re, w.x, -(a.im * wi));
+    r.im = wf_fma(a.im, w.x, a.re * wi);
+    return r;
+}
+
+/* Phase A: x the inputs x[g + R3 m], outputs to row[g + R3 n], n < R1 R2. */
+template <int N, int SIGN>
+__device__ __forceinline__ void wf_rx_phase_a(const wfc *x, wfc *row, const wf_real2 *__restrict__ tw, int g) {
+    constexpr int R1 = wf_radix_of(N, 0), R2 = wf_radix_of(N, 1), R3 = wf_rx_b(N), NA = R1 * R2;
+    static_assert(NA == wf_rx_a(N) && R3 == wf_radix_of(N, 2) && NA * R3 == N, "three-radix plan");
+    wf_real2 wt[NA]; /* the last radix's twiddles W_N^{g n} */
+#pragma unroll
+    for (int n = 1; n < NA; n++) wt[n] = tw[g * n];
+    wfc v[R2][R1];
+#pragma unroll
+    for (int r = 0; r < R2; r++) {
+        wfc in[R1];
+#pragma unroll
+        for (int s = 0; s < R1; s++) in[s] = x[r + R2 * s];
+        wf_dft_reg<R1, N / R1, SIGN>(in, tw, [&](int q, wfc y) { v[r][q] = y; });
+    }
+#pragma unroll
+    for (int kq = 0; kq < R1; kq++) {
+        wfc in[R2];
+#pragma unroll
+        for (int r = 0; r < R2; r++) in[r] = (r && kq) ? wf_twiddle<SIGN>(v[r][kq], tw[kq * r * R3]) : v[r][kq];
+        wf_dft_reg<R2, N / R2, SIGN>(in, tw, [&](int q, wfc y) {
+            const int n = kq + R1 * q;
+            row[g + R3 * n] = n ? wf_twiddle<SIGN>(y, wt[n]) : y;
+        });
+    }
+}
+/* Phase B: row[j R3 + r], r < R3 (phase A's outputs n = j) -> out(k, X_k), k = j + R1 R2 q. */
+template <int N, int SIGN, class Out>
+__device__ __forceinline__ void wf_rx_phase_b(const wfc *row, const wf_real2 *__restrict__ tw, int j, Out &&out) {
+    constexpr int R3 = wf_rx_b(N), NA = wf_rx_a(N);
+    wfc x[R3];
+#pragma unroll
+    for (int r = 0; r < R3; r++) x[r] = row[j * R3 + r];
+    wf_dft_reg<R3, N / R3, SIGN>(x, tw, [&](int q, wfc y) { out(j + NA * q, y); });
+}
 #endif
 
 #if defined(__HIPCC__)

@@ -151,7 +151,9 @@ struct WfHostFlag {
 #ifndef WF_FX_PAIRS
 #define WF_FX_PAIRS 4
 #endif
-__host__ __device__ constexpr int wf_pairs_for(int n) { return (n <= 300) ? WF_FX_PAIRS : 2; }
+__host__ __device__ constexpr int wf_pairs_for(int n) {
+    return (WF_MIXED && n == 255) ? 8 : (n <= 300) ? WF_FX_PAIRS : 2;
+}
 /* lengths with a compile-time plan */
 __host__ __device__ constexpr bool wf_planned(int n) { return n == 63 || n == 127 || n == 255 || n == 511; }
 #define WF_FY_COLS 4

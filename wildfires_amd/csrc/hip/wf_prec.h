@@ -40,6 +40,9 @@ typedef float2 wf_real2;
 typedef double wf_real;
 typedef double2 wf_real2;
 #endif
+/* one rounding, where a contraction is not left to the compiler */
+__device__ __forceinline__ float wf_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double wf_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 }  // namespace WF_NS
 
 #define WR(x) ((wf_real)(x))

@@ -36,15 +36,60 @@ namespace WF_NS {
 /* FP32 chunks of 8 levels: 8 waves per SIMD, so that two 16-wave workgroups
  * share a CU (256x256x128: 512 workgroups, one round of them) */
 #define WF_THOMAS_ATTR(LC) __attribute__((amdgpu_waves_per_eu((WF_MIXED && (LC) == 8) ? 8 : 4)))
+#define WF_FX_AHEAD 1
 #define WF_NX_SHORT 300
 template <int NX>
 struct WfFx {
     static constexpr int LEN = (NX > 0) ? NX : (NX == 0) ? WF_NX_SHORT : 1024;
     static constexpr int PAIRS = wf_pairs_for(LEN);
-    static constexpr int PER = (PAIRS * LEN + WF_NT - 1) / WF_NT;
+    static constexpr bool RX = NX > 0 && wf_rx_a(NX) != 0; /* register form of the plan */
+    /* compile-time lengths (2^m - 1): a row of LEN + 1 lanes per row pair, so
+     * that the rows of a wavefront, and with them every address but the
+     * column, are uniform; other lengths are packed */
+    static constexpr bool UNI = NX > 0;
+    static_assert(!UNI || (((NX + 1) & NX) == 0 && PAIRS * (NX + 1) % WF_NT == 0), "whole rows of lanes");
+    static constexpr int PER = (PAIRS * (UNI ? NX + 1 : LEN) + WF_NT - 1) / WF_NT;
+    /* LDS stride of a sequence: the register form's rows are 16 banks apart */
+    __device__ __forceinline__ static int stride(int n) { return RX ? NX + 9 : n; }
 };
-/* Transform of the PAIRS sequences in buf (compile-time plan when NX > 0, else
- * the run-time radices with scratch buffer bufb).  Returns the result buffer. */
+/* Element pi of this thread among the PAIRS rows of length nx: row pair s and
+ * column i, clamped to the last; true where it is one. */
+template <int NX>
+__device__ __forceinline__ bool wf_fx_elem(int pi, int nx, const WfDiv &by_nx, int *s, int *i) {
+    const int t = (int)threadIdx.x + pi * WF_NT;
+    if constexpr (WfFx<NX>::UNI) {
+        const int x = t & NX;
+        *s = __builtin_amdgcn_readfirstlane(t) / (NX + 1);
+        *i = min(x, NX - 1);
+        return x < NX;
+    } else {
+        const int n = WfFx<NX>::PAIRS * nx, tc = min(t, n - 1);
+        *s = by_nx(tc);
+        *i = tc - *s * nx;
+        return t < n;
+    }
+}
+/* F at an even ky and the next of a kx column: the spectra of a row pair */
+struct alignas(2 * sizeof(wf_real2)) WfPairF {
+    wf_real2 a, b;
+};
+/* Transform of the PAIRS sequences in buf: the register form of the plan from
+ * phase A's values on, the in-place plan (NX > 0), or the run-time radices with
+ * scratch buffer bufb; tw: twx for the first, else the table in LDS.  Returns
+ * the result buffer; ends with a barrier. */
+template <int NX, int SIGN>
+__device__ __forceinline__ wfc *wf_rx_finish(wfc *buf, wfc *bufb, const wf_real2 *__restrict__ twx) {
+    constexpr int PAIRS = WfFx<NX>::PAIRS, NA = wf_rx_a(NX);
+    static_assert(PAIRS * wf_rx_b(NX) <= WF_NT && PAIRS * NA <= WF_NT, "a thread takes one DFT of a phase");
+    __syncthreads();
+    if (threadIdx.x < PAIRS * NA) {
+        const int s = threadIdx.x / NA, j = threadIdx.x - s * NA;
+        const int o = s * WfFx<NX>::stride(NX);
+        wf_rx_phase_b<NX, SIGN>(buf + o, twx, j, [&](int k, wfc X) { bufb[o + k] = X; });
+    }
+    __syncthreads();
+    return bufb;
+}
 template <int NX>
 __device__ __forceinline__ wfc *wf_transform(wfc *buf, wfc *bufb, int n, const int *rad, const wfc *tw) {
     constexpr int PAIRS = WfFx<NX>::PAIRS;
@@ -87,71 +132,115 @@ __global__ __launch_bounds__(WF_NT) void k_iter_check(WfSpectral sp, double tol,
  * half-spectrum into F[k][kx][j].  NX > 0 selects the compile-time plan. */
 template <int NX, int MODE>
 __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectral &sp, const WfState &Ys,
-                                               const WfState &Yn, const wf_real *p, int block, int nblocks) {
+                                               const WfState &Yn, const wf_real *p, int block, int nblocks,
+                                               const wf_real2 *__restrict__ twx) {
     if (MODE != WF_F_TOP && sp.ctl->done) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
     constexpr int PAIRS = WfFx<NX>::PAIRS, PER = WfFx<NX>::PER;
-    const int nx = (NX > 0) ? NX : sp.nx;
+    constexpr bool RX = WfFx<NX>::RX;
+    const int nx = (NX > 0) ? NX : sp.nx, S = WfFx<NX>::stride(nx);
     const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
-    wfc *tw = smem, *bufa = smem + nx, *bufb = bufa + PAIRS * nx;
+    wfc *tw = smem, *bufa = RX ? smem : smem + nx, *bufb = bufa + PAIRS * S;
     int g, ks;
     wf_tile_decode_at(block, nblocks, sp.ngroups, (MODE == WF_F_TOP) ? 1 : sp.nz - 1, &g, &ks);
     const int k = (MODE == WF_F_TOP) ? c.Nz - 1 : 1 + ks;
     const int j0 = 2 * g * PAIRS;
-    for (int t = threadIdx.x; t < nx; t += blockDim.x) tw[t] = *(const wfc *)&sp.twx[t];
+    if constexpr (!RX)
+        for (int t = threadIdx.x; t < nx; t += blockDim.x) tw[t] = *(const wfc *)&sp.twx[t];
     if (NX <= 0 && threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
     const WfDiv by_nx(nx);
-    /* one row pair per batch: both cells' loads unconditional (indices clamped
-     * to a valid node, padding results dropped), so a batch is one basic block
-     * with all 28 loads in flight; the scheduling barrier keeps the batches
-     * apart, which bounds the registers */
+#if !WF_MIXED
+    if constexpr (MODE == WF_F_ITER && WfFx<NX>::UNI) {
+        /* What bounds this pass in FP64 is the cache's data path: 18 values a
+         * row pair by wf_pair_load against 30 node by node.  A row pair per
+         * batch, WF_FX_AHEAD batches of loads in flight before the one that is
+         * worked on, which the scheduling barriers keep so.  us at
+         * 256x256x128: node by node 76, with none ahead 69, one 67.5, two
+         * 68.4.  FP32, whose input is half of that, gains nothing (32.4-33.9
+         * against 32.7). */
+        const wf_real dzc = c.zc[WF_ZC * k + WF_Z_DZC];
+        WfPairIn v[PER];
+        const auto load = [&](int pi) {
+            int s, i;
+            (void)wf_fx_elem<NX>(pi, nx, by_nx, &s, &i);
+            wf_pair_load(c, sp.A, sp.rho, p, i, min(j0 + 2 * s, ny - 1), k, v[pi]);
+        };
 #pragma unroll
-    for (int pi = 0; pi < PER; pi++) {
-        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
-        const int t = threadIdx.x + pi * WF_NT;
-        if constexpr (MODE != WF_F_FIRST) {
-            const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
-            const int s = (NX > 0) ? tc / nx : by_nx(tc), i = tc - s * nx;
-            const int ja = j0 + 2 * s, jb = ja + 1;
-            const wf_real fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (ja < ny) ? ja : ny - 1, k);
-            const wf_real fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (jb < ny) ? jb : ny - 1, k);
-            if (t < PAIRS * nx) {
-                bufa[t].re = (ja < ny) ? fa : WR(0.0);
-                bufa[t].im = (jb < ny) ? fb : WR(0.0);
-            }
+        for (int pi = 0; pi < PER + WF_FX_AHEAD; pi++) {
+            if (pi < PER) load(pi);
             __builtin_amdgcn_sched_barrier(0);
-        } else if (t < PAIRS * nx) {
-            const int s = (NX > 0) ? t / nx : by_nx(t), i = t - s * nx;
+            if (pi < WF_FX_AHEAD) continue;
+            const int po = pi - WF_FX_AHEAD;
+            int s, i;
+            const bool ok = wf_fx_elem<NX>(po, nx, by_nx, &s, &i);
             const int ja = j0 + 2 * s, jb = ja + 1;
-            wf_real fa = WR(0.0), fb = WR(0.0);
-            if (ja < ny) fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, ja, k);
-            if (jb < ny) fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, jb, k);
-            bufa[t].re = fa;
-            bufa[t].im = fb;
+            wf_real fa, fb;
+            wf_pair_eval(c, v[po], i, dzc, &fa, &fb);
+            if (ok) bufa[s * S + i] = wfc{(ja < ny) ? fa : WR(0.0), (jb < ny) ? fb : WR(0.0)};
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else
+#endif
+    {
+        /* one row pair per batch: both cells' loads unconditional (indices clamped
+         * to a valid node, padding results dropped), so a batch is one basic block
+         * with all 28 loads in flight; the scheduling barrier keeps the batches
+         * apart, which bounds the registers */
+#pragma unroll
+        for (int pi = 0; pi < PER; pi++) {
+            if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
+            int s, i;
+            const bool ok = wf_fx_elem<NX>(pi, nx, by_nx, &s, &i);
+            const int ja = j0 + 2 * s, jb = ja + 1;
+            if constexpr (MODE != WF_F_FIRST) {
+                const wf_real fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (ja < ny) ? ja : ny - 1, k);
+                const wf_real fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, (jb < ny) ? jb : ny - 1, k);
+                if (ok) bufa[s * S + i] = wfc{(ja < ny) ? fa : WR(0.0), (jb < ny) ? fb : WR(0.0)};
+                __builtin_amdgcn_sched_barrier(0);
+            } else if (ok) {
+                wf_real fa = WR(0.0), fb = WR(0.0);
+                if (ja < ny) fa = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, ja, k);
+                if (jb < ny) fb = wf_fx_input<MODE>(c, sp, Ys, Yn, p, i, jb, k);
+                bufa[s * S + i] = wfc{fa, fb};
+            }
         }
     }
     __syncthreads();
-    wfc *res = wf_transform<NX>(bufa, bufb, nx, rad, tw);
+    wfc *res;
+    if constexpr (RX) {
+        constexpr int NA = wf_rx_a(NX), NB = wf_rx_b(NX);
+        if (threadIdx.x < PAIRS * NB) {
+            const int s = threadIdx.x / NB, g = threadIdx.x - s * NB;
+            wfc x[NA]; /* phase A writes where it read */
+#pragma unroll
+            for (int m = 0; m < NA; m++) x[m] = bufa[s * S + g + NB * m];
+            wf_rx_phase_a<NX, -1>(x, bufa + s * S, twx, g);
+        }
+        res = wf_rx_finish<NX, -1>(bufa, bufb, twx);
+    } else {
+        res = wf_transform<NX>(bufa, bufb, nx, rad, tw);
+    }
+    /* a thread unpacks both rows of a pair */
     wf_real2 *dst = (MODE == WF_F_TOP) ? sp.Ptop : sp.F + (long)k * hx * ldj;
-    constexpr int rows = 2 * PAIRS;
-    for (int t = threadIdx.x; t < rows * hx; t += blockDim.x) {
-        const int jl = t % rows, r = t / rows;
-        const int j = j0 + jl;
-        if (j >= ny) continue;
-        const int s = jl >> 1;
+    for (int t = threadIdx.x; t < PAIRS * hx; t += WF_NT) {
+        const int s = t % PAIRS, r = t / PAIRS, ja = j0 + 2 * s;
         const int rm = (r == 0) ? 0 : nx - r;
         wfc A, B;
-        wf_unpack_pair(res[s * nx + r], res[s * nx + rm], &A, &B);
-        dst[(long)r * ldj + j] = (jl & 1) ? wf_make2(B.re, B.im) : wf_make2(A.re, A.im);
+        wf_unpack_pair(res[s * S + r], res[s * S + rm], &A, &B);
+        wf_real2 *d = dst + (unsigned)(r * ldj + ja);
+        if (ja + 1 < ny)
+            *(WfPairF *)d = WfPairF{wf_make2(A.re, A.im), wf_make2(B.re, B.im)};
+        else if (ja < ny)
+            *d = wf_make2(A.re, A.im);
     }
 }
 template <int NX, int MODE>
 __global__ __launch_bounds__(WF_NT) void k_rhs_fx(WfConst c, WfSpectral sp, WfState Ys, WfState Yn,
                                                   const wf_real *p, double tol, double rtol, int check,
-                                                  int max_iter) {
+                                                  int max_iter, const wf_real2 *__restrict__ twx) {
     const int b = wf_checked_block(sp, tol, rtol, check, max_iter);
-    if (b >= 0) wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p, b, (int)gridDim.x - (check >= 0));
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p, b, (int)gridDim.x - (check >= 0), twx);
 }
 
 /* P2/P4: y-transform of sp.fy_cols kx columns (each contiguous over ky) of
@@ -614,42 +703,43 @@ __global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) __attribute__((amdgpu_wa
  * the group that holds j = 0). */
 template <int NX>
 __device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectral &sp, wf_real *p, wfc *smem,
-                                                  const int *rad, int g, int k, double &dmax, double &pabs) {
+                                                  const int *rad, int g, int k, wf_real &dmax, wf_real &pabs,
+                                               const wf_real2 *__restrict__ twx) {
     constexpr int PAIRS = WfFx<NX>::PAIRS, PER = WfFx<NX>::PER;
     constexpr int PERY = (WfFx<NX>::LEN + 1 + WF_NT - 1) / WF_NT; /* row j = Ny-1: i = 0 .. Nx-1 */
-    const int nx = (NX > 0) ? NX : sp.nx;
+    constexpr bool RX = WfFx<NX>::RX;
+    const int nx = (NX > 0) ? NX : sp.nx, S = WfFx<NX>::stride(nx);
     const WfDiv by_nx(nx);
     const int ny = sp.ny, hx = sp.hx, ldj = sp.ldj;
     const int j0 = 2 * g * PAIRS;
     const wf_real2 *src = sp.F + (long)k * hx * ldj;
     const wf_real inv_scale = WR(1.0) / ((wf_real)nx * (wf_real)ny);
     const int tid = threadIdx.x;
-    wfc *tw = smem, *buf = smem + nx;
-    /* loads: half spectra (thread t -> pair t % PAIRS, bin t / PAIRS, so
-     * consecutive threads read consecutive ky of one kx column) */
-    wf_real2 xa[PER], xb[PER];
+    wfc *tw = smem, *buf = RX ? smem : smem + nx;
+    /* loads: half spectra of a row pair (thread t -> pair t % PAIRS and bin, or
+     * phase A's block, t / PAIRS, so consecutive threads read consecutive ky of
+     * one kx column) */
+    constexpr int NA = RX ? wf_rx_a(NX) : PER, NB = RX ? wf_rx_b(NX) : 1;
+    WfPairF xp[NA];
+    const int sA = tid % PAIRS, gA = tid / PAIRS, jA = j0 + 2 * sA;
+    const int jl = min(jA, (ny - 1) & ~1);
 #pragma unroll
-    for (int pi = 0; pi < PER; pi++) {
-        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
-        const int t = tid + pi * WF_NT;
-        const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
-        const int s = tc % PAIRS, r = tc / PAIRS;
-        const int ja = j0 + 2 * s, jb = ja + 1;
+    for (int m = 0; m < NA; m++) {
+        if (NX <= 0 && m * WF_NT >= PAIRS * nx) break;
+        const int r = RX ? min(gA, NB - 1) + NB * m : min(gA + m * (WF_NT / PAIRS), nx - 1);
         const int rr = (r >= hx) ? nx - r : r;
-        xa[pi] = src[(long)rr * ldj + ((ja < ny) ? ja : ny - 1)];
-        xb[pi] = src[(long)rr * ldj + ((jb < ny) ? jb : ny - 1)];
+        xp[m] = *(const WfPairF *)&src[(unsigned)(rr * ldj + jl)];
     }
-    /* old p of the unique nodes (thread t -> pair t / NX, i = t % NX) */
+    /* old p of the unique nodes */
     wf_real pa[PER], pb[PER];
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
         if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
-        const int t = tid + pi * WF_NT;
-        const int tc = (t < PAIRS * nx) ? t : PAIRS * nx - 1;
-        const int s = (NX > 0) ? tc / nx : by_nx(tc), i = tc - s * nx;
+        int s, i;
+        (void)wf_fx_elem<NX>(pi, nx, by_nx, &s, &i);
         const int ja = j0 + 2 * s, jb = ja + 1;
-        pa[pi] = p[wf_q(c, i, (ja < ny) ? ja : ny - 1, k)];
-        pb[pi] = p[wf_q(c, i, (jb < ny) ? jb : ny - 1, k)];
+        pa[pi] = wf_ldp(p + wf_q(c, 0, (ja < ny) ? ja : ny - 1, k), (unsigned)i);
+        pb[pi] = wf_ldp(p + wf_q(c, 0, (jb < ny) ? jb : ny - 1, k), (unsigned)i);
     }
     /* old p of the duplicates: column i = Nx-1 of the group's rows, and
      * row j = Ny-1 (i = 0 .. Nx-1) when the group holds j = 0 */
@@ -663,62 +753,66 @@ __device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectra
             pdy[pi] = p[wf_q(c, (i <= nx) ? i : nx, c.Ny - 1, k)];
         }
     }
-    for (int t = tid; t < nx; t += WF_NT) {
-        const wf_real2 w = sp.twx[t];
-        tw[t].re = w.x;
-        tw[t].im = -w.y;
-    }
+    /* entry m of this thread as a bin of the packed pair */
+    const auto packed = [&](int m, bool conj) {
+        const wfc A = {xp[m].a.x, xp[m].a.y};
+        wfc B = {WR(0.0), WR(0.0)};
+        if (jA + 1 < ny) B = wfc{xp[m].b.x, xp[m].b.y};
+        return wf_pack_pair(A, B, conj);
+    };
+    if constexpr (RX) {
+        if (tid < PAIRS * NB) {
+            wfc x[NA];
 #pragma unroll
-    for (int pi = 0; pi < PER; pi++) {
-        if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
-        const int t = tid + pi * WF_NT;
-        const int s = t % PAIRS, r = t / PAIRS;
-        const int ja = j0 + 2 * s, jb = ja + 1;
-        if (t < PAIRS * nx) {
-            wfc A = {WR(0.0), WR(0.0)}, B = {WR(0.0), WR(0.0)};
-            if (ja < ny) {
-                A.re = xa[pi].x;
-                A.im = xa[pi].y;
-                if (jb < ny) {
-                    B.re = xb[pi].x;
-                    B.im = xb[pi].y;
-                }
-            }
-            buf[s * nx + r] = wf_pack_pair(A, B, r >= hx);
+            for (int m = 0; m < NA; m++) x[m] = packed(m, gA + NB * m >= NX / 2 + 1);
+            wf_rx_phase_a<NX, 1>(x, buf + sA * S, twx, gA);
         }
+        buf = wf_rx_finish<NX, 1>(buf, buf + PAIRS * S, twx);
+    } else {
+        for (int t = tid; t < nx; t += WF_NT) {
+            const wf_real2 w = sp.twx[t];
+            tw[t].re = w.x;
+            tw[t].im = -w.y;
+        }
+#pragma unroll
+        for (int m = 0; m < NA; m++) {
+            if (NX <= 0 && m * WF_NT >= PAIRS * nx) break;
+            const int r = gA + m * (WF_NT / PAIRS);
+            if (r < nx) buf[sA * nx + r] = packed(m, r >= hx);
+        }
+        __syncthreads();
+        buf = wf_transform<NX>(buf, buf + PAIRS * nx, nx, rad, tw);
     }
-    __syncthreads();
-    buf = wf_transform<NX>(buf, buf + PAIRS * nx, nx, rad, tw);
     /* unique nodes */
 #pragma unroll
     for (int pi = 0; pi < PER; pi++) {
         if (NX <= 0 && pi * WF_NT >= PAIRS * nx) break;
-        const int t = tid + pi * WF_NT;
-        const int s = (NX > 0) ? t / nx : by_nx(t), i = t - s * nx;
+        int s, i;
+        const bool ok = wf_fx_elem<NX>(pi, nx, by_nx, &s, &i);
         const int ja = j0 + 2 * s, jb = ja + 1;
-        if (t < PAIRS * nx) {
-            const wfc v = buf[s * nx + i];
+        if (ok) {
+            const wfc v = buf[s * S + i];
             if (ja < ny) {
                 const wf_real pv = v.re * inv_scale;
-                const double d = (double)fabs(pv - pa[pi]);
+                const wf_real d = fabs(pv - pa[pi]);
                 dmax = (d > dmax) ? d : dmax;
-                if constexpr (WF_MIXED) pabs = ((double)fabs(pv) > pabs) ? (double)fabs(pv) : pabs;
-                p[wf_q(c, i, ja, k)] = pv;
+                if constexpr (WF_MIXED) pabs = (fabs(pv) > pabs) ? fabs(pv) : pabs;
+                (p + wf_q(c, 0, ja, k))[(unsigned)i] = pv;
             }
             if (jb < ny) {
                 const wf_real pv = v.im * inv_scale;
-                const double d = (double)fabs(pv - pb[pi]);
+                const wf_real d = fabs(pv - pb[pi]);
                 dmax = (d > dmax) ? d : dmax;
-                if constexpr (WF_MIXED) pabs = ((double)fabs(pv) > pabs) ? (double)fabs(pv) : pabs;
-                p[wf_q(c, i, jb, k)] = pv;
+                if constexpr (WF_MIXED) pabs = (fabs(pv) > pabs) ? fabs(pv) : pabs;
+                (p + wf_q(c, 0, jb, k))[(unsigned)i] = pv;
             }
         }
     }
     /* duplicate column i = Nx-1 of rows j0 .. j0 + 2 PAIRS - 1 (value of i = 0) */
     if (tid < 2 * PAIRS && jr < ny) {
-        const wfc v = buf[(tid >> 1) * nx];
+        const wfc v = buf[(tid >> 1) * S];
         const wf_real pv = ((tid & 1) ? v.im : v.re) * inv_scale;
-        const double d = (double)fabs(pv - pdx);
+        const wf_real d = fabs(pv - pdx);
         dmax = (d > dmax) ? d : dmax;
         p[wf_q(c, c.Nx - 1, jr, k)] = pv;
     }
@@ -729,7 +823,7 @@ __device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectra
             const int i = tid + pi * WF_NT;
             if (i <= nx) {
                 const wf_real pv = buf[(i < nx) ? i : 0].re * inv_scale;
-                const double d = (double)fabs(pv - pdy[pi]);
+                const wf_real d = fabs(pv - pdy[pi]);
                 dmax = (d > dmax) ? d : dmax;
                 p[wf_q(c, i, c.Ny - 1, k)] = pv;
             }
@@ -738,34 +832,37 @@ __device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectra
 }
 
 template <int NX>
-__device__ __forceinline__ void wf_inv_fx_body(const WfConst &c, const WfSpectral &sp, wf_real *p) {
+__device__ __forceinline__ void wf_inv_fx_body(const WfConst &c, const WfSpectral &sp, wf_real *p,
+                                               const wf_real2 *__restrict__ twx) {
     if (sp.ctl->done) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
-    double dmax = 0.0, pabs = 0.0;
     if (blockIdx.x == gridDim.x - 1) {
-        wf_top_duplicates(c, p, dmax);
-        wf_block_max_store(dmax, &sp.pmax[blockIdx.x]);
+        double dtop = 0.0;
+        wf_top_duplicates(c, p, dtop);
+        wf_block_max_store(dtop, &sp.pmax[blockIdx.x]);
         if constexpr (WF_MIXED) {
             __syncthreads();
-            wf_block_max_store(pabs, &sp.pmax[sp.npmax + blockIdx.x]);
+            wf_block_max_store(0.0, &sp.pmax[sp.npmax + blockIdx.x]);
         }
         return;
     }
+    wf_real dmax = WR(0.0), pabs = WR(0.0);
     /* the tiles are blocks 0 .. gridDim.x - 2 (the last block is the one above) */
     int g, k;
     wf_tile_decode_at((int)blockIdx.x, (int)gridDim.x - 1, sp.ngroups, sp.nz, &g, &k);
     if (NX <= 0 && threadIdx.x < WF_MAX_RADICES) rad[threadIdx.x] = sp.radx[threadIdx.x];
-    wf_inv_fx_rows<NX>(c, sp, p, smem, rad, g, k, dmax, pabs);
-    wf_block_max_store(dmax, &sp.pmax[blockIdx.x]);
+    wf_inv_fx_rows<NX>(c, sp, p, smem, rad, g, k, dmax, pabs, twx);
+    wf_block_max_store((double)dmax, &sp.pmax[blockIdx.x]);
     if constexpr (WF_MIXED) {
         __syncthreads();
-        wf_block_max_store(pabs, &sp.pmax[sp.npmax + blockIdx.x]);
+        wf_block_max_store((double)pabs, &sp.pmax[sp.npmax + blockIdx.x]);
     }
 }
 template <int NX>
-__global__ __launch_bounds__(WF_NT) void k_inv_fx(WfConst c, WfSpectral sp, wf_real *p) {
-    wf_inv_fx_body<NX>(c, sp, p);
+__global__ __launch_bounds__(WF_NT) void k_inv_fx(WfConst c, WfSpectral sp, wf_real *p,
+                                                  const wf_real2 *__restrict__ twx) {
+    wf_inv_fx_body<NX>(c, sp, p, twx);
 }
 
 /* ------------------------------------------------- batched size classes ---- */
@@ -781,10 +878,11 @@ __global__ void k_iter_reset_batch(const WfPressItem *__restrict__ tab) {
 }
 
 template <int NX, int MODE>
-__global__ __launch_bounds__(WF_NT) void k_rhs_fx_batch(const WfPressItem *__restrict__ tab, int check) {
+__global__ __launch_bounds__(WF_NT) void k_rhs_fx_batch(const WfPressItem *__restrict__ tab, int check,
+                                                        const wf_real2 *__restrict__ twx) {
     const WfPressItem it = wf_press_load(tab);
     const int b = wf_checked_block(it.sp, it.tol, it.rtol, check, it.max_iter);
-    if (b >= 0) wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, (int)gridDim.x - (check >= 0));
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, (int)gridDim.x - (check >= 0), twx);
 }
 
 /* twy: the class's y twiddle table (it depends on ny alone, so every member's
@@ -813,9 +911,10 @@ __global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) __attribute__((amdgpu_wa
 #endif
 
 template <int NX>
-__global__ __launch_bounds__(WF_NT) void k_inv_fx_batch(const WfPressItem *__restrict__ tab) {
+__global__ __launch_bounds__(WF_NT) void k_inv_fx_batch(const WfPressItem *__restrict__ tab,
+                                                        const wf_real2 *__restrict__ twx) {
     const WfPressItem it = wf_press_load(tab);
-    wf_inv_fx_body<NX>(it.c, it.sp, it.p);
+    wf_inv_fx_body<NX>(it.c, it.sp, it.p, twx);
 }
 
 __global__ __launch_bounds__(WF_NT) void k_iter_check_batch(const WfPressItem *__restrict__ tab, int m) {
@@ -828,6 +927,7 @@ __global__ __launch_bounds__(WF_NT) void k_iter_check_batch(const WfPressItem *_
 /* dynamic LDS of an x-transform kernel: twiddles + one buffer (compile-time
  * plan, in place) or two buffers (run-time radices) */
 static size_t wf_fx_lds(int n, int nseq) {
+    if (wf_rx_a(n)) return sizeof(wfc) * (size_t)(n + 9) * 2 * (size_t)nseq;
     return sizeof(wfc) * (size_t)n * (1 + (wf_planned(n) ? 1 : 2) * (size_t)nseq);
 }
 
@@ -901,16 +1001,16 @@ hipError_t wf_launch_pressure_rhs_fx(const WfConst &c, const WfSpectral &sp, con
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
     switch (mode) {
         case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
-                                        check, max_iter);
+                                        check, max_iter, (const wf_real2 *)sp.twx);
             break;
         case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
-                                        check, max_iter);
+                                        check, max_iter, (const wf_real2 *)sp.twx);
             break;
         case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
-                                        check, max_iter);
+                                        check, max_iter, (const wf_real2 *)sp.twx);
             break;
         default: WF_DISPATCH_NM(k_rhs_fx, sp.nx, WF_F_TOP, grd, dim3(WF_NT), lds, s, c, sp, Ys, Yn, p, tol, rtol,
-                                        check, max_iter);
+                                        check, max_iter, (const wf_real2 *)sp.twx);
             break;
     }
     return hipGetLastError();
@@ -963,7 +1063,7 @@ hipError_t wf_launch_iter_check(const WfSpectral &sp, double tol, double rtol, i
 hipError_t wf_launch_inverse_fx(const WfConst &c, const WfSpectral &sp, wf_real *p, hipStream_t s) {
     dim3 grd((unsigned)sp.npmax);
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
-    WF_DISPATCH_N(sp.nx, k_inv_fx, grd, dim3(WF_NT), lds, s, c, sp, p);
+    WF_DISPATCH_N(sp.nx, k_inv_fx, grd, dim3(WF_NT), lds, s, c, sp, p, (const wf_real2 *)sp.twx);
     return hipGetLastError();
 }
 
@@ -986,9 +1086,15 @@ hipError_t wf_launch_pressure_rhs_fx_batch(const WfSpectral &sp, const WfPressIt
     dim3 grd((unsigned)(sp.ngroups * nslabs + (check >= 0)), 1, nm);
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
     switch (mode) {
-        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, tab, check); break;
-        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, tab, check); break;
-        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, tab, check); break;
+        case WF_F_ITER: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_ITER, grd, dim3(WF_NT), lds, s, tab, check,
+                                        (const wf_real2 *)sp.twx);
+            break;
+        case WF_F_FIRST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_FIRST, grd, dim3(WF_NT), lds, s, tab, check,
+                                        (const wf_real2 *)sp.twx);
+            break;
+        case WF_F_CONST: WF_DISPATCH_NM(k_rhs_fx_batch, sp.nx, WF_F_CONST, grd, dim3(WF_NT), lds, s, tab, check,
+                                        (const wf_real2 *)sp.twx);
+            break;
         default: return hipErrorInvalidValue; /* the top plane is solo only */
     }
     return hipGetLastError();
@@ -1032,7 +1138,7 @@ hipError_t wf_launch_thomas_batch(const WfSpectral &sp, const WfPressItem *tab, 
 hipError_t wf_launch_inverse_fx_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s) {
     dim3 grd((unsigned)sp.npmax, 1, nm);
     size_t lds = wf_fx_lds(sp.nx, sp.fx_pairs);
-    WF_DISPATCH_N(sp.nx, k_inv_fx_batch, grd, dim3(WF_NT), lds, s, tab);
+    WF_DISPATCH_N(sp.nx, k_inv_fx_batch, grd, dim3(WF_NT), lds, s, tab, (const wf_real2 *)sp.twx);
     return hipGetLastError();
 }
 

@@ -137,6 +137,79 @@ __device__ __forceinline__ wf_real wf_f_pgrad(const WfConst &c, const wf_real *r
     return (rhox * px + rhoy * py + rhoz * pz) / rho;
 }
 
+#if !WF_MIXED
+/* v of the lane below (lane 0: edge) and of the lane above (lane 63: edge) */
+__device__ __forceinline__ double wf_lane_below(double v, double edge) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x138, 0xf, 0xf, false),
+        __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double wf_lane_above(double v, double edge) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x130, 0xf, 0xf, false),
+        __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x130, 0xf, 0xf, false));
+}
+
+/* The later iterations' input on the pair of nodes (i, ja), (i, ja + 1) of a
+ * wavefront whose lanes hold consecutive columns i from a multiple of 64 on
+ * (those past the last clamped to it) of one row pair: the two rows are each
+ * other's y-neighbours (past the last row the second is row 0, and its result
+ * of no meaning), the x-neighbours come from the lanes beside, except at the
+ * ends of the wavefront and of the row. */
+struct WfPairIn {
+    wf_real A[2], a[2], b[2], ym[2], yp[2], azm[2], azp[2], bzm[2], bzp[2], ea[2], eb[2];
+};
+__device__ __forceinline__ void wf_pair_load(const WfConst &c, const wf_real *A, const wf_real *rho_n, const wf_real *p,
+                                             int i, int ja, int k, WfPairIn &v) {
+    const unsigned Nx = (unsigned)c.Nx, P = (unsigned)c.plane, zrow = (unsigned)c.Ny * (unsigned)k;
+    const int jb = wf_wrap_p(ja, 1, c.Ny);
+    const unsigned ra = Nx * (zrow + (unsigned)ja), rb = Nx * (zrow + (unsigned)jb);
+    const unsigned rm = Nx * (zrow + (unsigned)wf_wrap_m(ja, 1, c.Ny)), rp = Nx * (zrow + (unsigned)wf_wrap_p(jb, 1, c.Ny));
+    const int lane = (int)__lane_id();
+    const unsigned ie = (unsigned)((lane == 0) ? wf_wrap_m(i, 1, c.Nx) : wf_wrap_p(i, 1, c.Nx));
+    const wf_real *f[2] = {rho_n, p};
+    v.A[0] = wf_ldp(A + ra, i);
+    v.A[1] = wf_ldp(A + rb, i);
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        v.a[n] = wf_ldp(f[n] + ra, i);
+        v.b[n] = wf_ldp(f[n] + rb, i);
+        v.ym[n] = wf_ldp(f[n] + rm, i);
+        v.yp[n] = wf_ldp(f[n] + rp, i);
+        v.azm[n] = wf_ldp(f[n] + (ra - P), i);
+        v.azp[n] = wf_ldp(f[n] + (ra + P), i);
+        v.bzm[n] = wf_ldp(f[n] + (rb - P), i);
+        v.bzp[n] = wf_ldp(f[n] + (rb + P), i);
+        v.ea[n] = v.eb[n] = WR(0.0);
+    }
+    if (lane == 0 || lane == 63 || i >= c.Nx - 2) {
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            v.ea[n] = wf_ldp(f[n] + ra, ie);
+            v.eb[n] = wf_ldp(f[n] + rb, ie);
+        }
+    }
+}
+/* wf_f_pgrad's operations, the contractions spelled out */
+__device__ __forceinline__ void wf_pair_eval(const WfConst &c, const WfPairIn &v, int i, wf_real dzc, wf_real *fa,
+                                             wf_real *fb) {
+    const bool last = i >= c.Nx - 2;
+    wf_real ax[2], ay[2], az[2], bx[2], by[2], bz[2];
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        const wf_real au = wf_lane_above(v.a[n], v.ea[n]), bu = wf_lane_above(v.b[n], v.eb[n]);
+        ax[n] = ((last ? v.ea[n] : au) - wf_lane_below(v.a[n], v.ea[n])) * c.inv2dx;
+        bx[n] = ((last ? v.eb[n] : bu) - wf_lane_below(v.b[n], v.eb[n])) * c.inv2dx;
+        ay[n] = (v.b[n] - v.ym[n]) * c.inv2dy;
+        by[n] = (v.yp[n] - v.a[n]) * c.inv2dy;
+        az[n] = (v.azp[n] - v.azm[n]) * dzc;
+        bz[n] = (v.bzp[n] - v.bzm[n]) * dzc;
+    }
+    *fa = v.A[0] + wf_fma(az[0], az[1], wf_fma(ay[0], ay[1], ax[0] * ax[1])) / v.a[0];
+    *fb = v.A[1] + wf_fma(bz[0], bz[1], wf_fma(by[0], by[1], bx[0] * bx[1])) / v.b[0];
+}
+#endif
+
 /* Maximum of the n partial maxima a[] (>= 0) over the workgroup, into *out
  * (16 independent loads per thread and pass, so one pass costs one memory
  * round trip; a plain strided loop waits for each load in turn). */
