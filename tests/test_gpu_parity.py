@@ -383,3 +383,25 @@ def test_compile_time_x_lengths(tmp_path, monkeypatch, precision, nx, ny, nz):
     print("%dx%dx%d %s rel %.2e" % (nx, ny, nz, precision, rel_l2(pg, po)), flush=True)
     assert rel_l2(pg, po) <= (1e-11 if precision == "fp64" else 2e-5)
     assert ig == io
+
+
+@pytest.mark.parametrize("nz", [129, 130, 257])
+def test_tridiagonal_chunks_fp64(tmp_path, nz):
+    """128 levels in chunks of 8, 129 and 256 in chunks of 16 (a component of
+    a system to a lane), on a grid whose solve keeps the two-factor
+    transforms: four solves of the iteration within 1e-11 of the oracle, the
+    bound of the other pressure tests."""
+    from oracle import oracle
+    from wildfires_amd import api
+    prm = make_params(tmp_path, "small_flat", Nx=64, Ny=256, Nz=nz, x_max=126.0, y_max=510.0, z_max=0.5 * (nz - 1),
+                      pressure_solver_iter=4)
+    y, p = perturbed_state(prm)
+    O = oracle.Oracle(prm.ptr)
+    y1 = y + prm.p.dt * O.phi(y)
+    with api.Solver(prm) as solver:
+        pg, _, ig = solver.pressure(y1, y, p)
+    po = p.copy()
+    _, io, _ = O.pressure(y1, y, po)
+    print("64x256x%d rel %.2e" % (nz, rel_l2(pg, po)), flush=True)
+    assert rel_l2(pg, po) <= 1e-11
+    assert ig == io

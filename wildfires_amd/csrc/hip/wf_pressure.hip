@@ -388,7 +388,10 @@ __global__ void k_pivots(WfSpectral sp, double *UB) {
  * their values finite and apart from the others. */
 template <typename TA, int NC>
 struct WfThomasLds {
-    TA v[WF_THOMAS_MAX_CHUNKS][64][NC], g[WF_THOMAS_MAX_CHUNKS][64];
+    struct alignas(NC * sizeof(TA)) V { /* one LDS access (two would meet in the banks) */
+        TA c[NC];
+    } v[WF_THOMAS_MAX_CHUNKS][64];
+    TA g[WF_THOMAS_MAX_CHUNKS][64];
 };
 template <int LC, typename TA, int NC>
 __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLds<TA, NC> &L, int j, int r,
@@ -402,25 +405,36 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
     const long row = (long)r * sp.ldj; /* uniform: a level's entries are at a scalar base + at */
     const unsigned jj = ok ? j : 0, at = 2 * jj + comp;
     const int k0 = w * LC;
+    /* the operands of the pivots first: their chain of divisions runs while the
+     * right-hand sides arrive */
+    TA u = w ? (TA)(sp.UB + row + w * slab)[jj] : (TA)sp.b0; /* pivot entering the chunk */
+    const TA K2 = wf_tab<TA>(sp.kx2, sp.kx2d, r) + wf_tab<TA>(sp.ky2, sp.ky2d, jj);
+    __builtin_amdgcn_sched_barrier(0);
     TA y[LC][NC], g[LC], ru[LC], pt[NC];
-#pragma unroll
-    for (int t = 0; t < LC; t++) {
+    const auto load = [&](int t) {
         int k = min(k0 + t, nz - 1);
         if (t == 0) k = max(k, 1); /* level 0 takes level 1's right-hand side */
 #pragma unroll
         for (int q = 0; q < NC; q++) y[t][q] = (TA)((const wf_real *)(sp.F + row + k * slab))[at + q];
+    };
+    /* FP64 (one workgroup per CU): a level's load before each level's
+     * divisions, so that the memory has work while a round computes (all
+     * first: 33.0 us against 31.8 at 256x256x128, 68 against 51 at 160 levels) */
+    constexpr bool SPREAD = sizeof(TA) * NC == 16;
+    if constexpr (!SPREAD) {
+#pragma unroll
+        for (int t = 0; t < LC; t++) load(t);
     }
 #pragma unroll
     for (int q = 0; q < NC; q++)
-        pt[q] = (k0 + LC >= nz) ? (TA)((const wf_real *)(sp.Ptop + row))[at + q] / (TA)sp.top_div : (TA)0.0;
-    TA u = w ? (TA)(sp.UB + row + w * slab)[jj] : (TA)sp.b0; /* pivot entering the chunk */
-    const TA K2 = wf_tab<TA>(sp.kx2, sp.kx2d, r) + wf_tab<TA>(sp.ky2, sp.ky2d, jj);
+        pt[q] = (k0 + LC >= nz) ? (TA)((const wf_real *)(sp.Ptop + row))[at + q] : (TA)0.0;
     const TA half_dz0 = (TA)0.5 * (TA)sp.dz0;
     const TA c0 = (TA)sp.c0a - half_dz0 * K2 - (TA)sp.c0b;
     const TA ck0 = w ? wf_tab<TA>(sp.tc, sp.tcd, k0) : c0; /* c_{k0} */
     /* the pivots u_k (wf_pivot_next's operations), L_k and 1/u_k */
 #pragma unroll
     for (int t = 0; t < LC; t++) {
+        if constexpr (SPREAD) load(t);
         const int km = (t > 0) ? k0 + t - 1 : max(k0 - 1, 0);
         const TA bk = -(K2 + wf_tab<TA>(sp.beta, sp.betad, k0 + t));
         const TA l = wf_tab<TA>(sp.ta, sp.tad, km) / u;
@@ -431,11 +445,14 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
             g[0] = w ? l : (TA)0.0;
         }
         ru[t] = (TA)1.0 / u;
+        if constexpr (SPREAD) __builtin_amdgcn_sched_barrier(0);
     }
+    __builtin_amdgcn_sched_barrier(0);
     /* forward elimination, entry value 0, coefficient G of the entry value */
     TA acc[NC], G = (TA)1.0;
 #pragma unroll
     for (int q = 0; q < NC; q++) {
+        if (k0 + LC >= nz) pt[q] = pt[q] / (TA)sp.top_div;
         acc[q] = (TA)0.0;
         y[0][q] = w ? y[0][q] : half_dz0 * y[0][q];
     }
@@ -449,8 +466,10 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
         }
         g[t] = G = -m * G;
     }
+    typename WfThomasLds<TA, NC>::V e;
 #pragma unroll
-    for (int q = 0; q < NC; q++) L.v[w][lane][q] = acc[q];
+    for (int q = 0; q < NC; q++) e.c[q] = acc[q];
+    L.v[w][lane] = e;
     L.g[w][lane] = G;
     __syncthreads();
     TA Y[NC];
@@ -459,8 +478,9 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
 #pragma unroll 4
     for (int s = 0; s < w; s++) {
         const TA gs = L.g[s][lane];
+        const auto vs = L.v[s][lane];
 #pragma unroll
-        for (int q = 0; q < NC; q++) Y[q] = L.v[s][lane][q] + gs * Y[q];
+        for (int q = 0; q < NC; q++) Y[q] = vs.c[q] + gs * Y[q];
     }
 #pragma unroll
     for (int t = 0; t < LC; t++)
@@ -479,7 +499,8 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
         g[t] = H = (-ck * ru[t]) * H;
     }
 #pragma unroll
-    for (int q = 0; q < NC; q++) L.v[w][lane][q] = xa[q];
+    for (int q = 0; q < NC; q++) e.c[q] = xa[q];
+    L.v[w][lane] = e;
     L.g[w][lane] = H;
     __syncthreads();
     TA X[NC];
@@ -488,8 +509,9 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
 #pragma unroll 4
     for (int s = C - 1; s > w; s--) {
         const TA hs = L.g[s][lane];
+        const auto vs = L.v[s][lane];
 #pragma unroll
-        for (int q = 0; q < NC; q++) X[q] = L.v[s][lane][q] + hs * X[q];
+        for (int q = 0; q < NC; q++) X[q] = vs.c[q] + hs * X[q];
     }
     if (!ok) return;
 #pragma unroll
@@ -517,9 +539,10 @@ __device__ __forceinline__ void wf_thomas_body(const WfSpectral &sp) {
      * halves are low_kx rows of workgroups before the kx columns'.  us, with
      * a complex FP64 system to a lane, 105 registers and a branch per level
      * before: 64x64x32 8.6 -> 5.3, 128x128x64 10.8 -> 8.2, 201x151x81 16 ->
-     * 13.8, 256x256x128 23.2 -> 20.5 (16.2 without the FP64 systems, whose
-     * extra workgroups there start when the first others end).  Both halves
-     * by one workgroup in turn: 9.5, 16.1, 20.7, 29.4. */
+     * 13.8, 256x256x128 23.2 -> 18.8 (16.2 without the FP64 systems, whose
+     * extra workgroups there start when the first others end); in FP64, all
+     * systems complex, 256x256x64 16.4 -> 15.4, 256x256x128 as before (32.4).
+     * Both halves by one workgroup in turn: 9.5, 16.1, 20.7, 29.4. */
     __shared__ union {
         WfThomasLds<float, 2> f;
         WfThomasLds<double, 1> d;
@@ -533,8 +556,15 @@ __device__ __forceinline__ void wf_thomas_body(const WfSpectral &sp) {
     else if (!second)
         wf_thomas_solve<LC, float, 2>(sp, L.f, jlo + lane, r, 0);
 #else
-    __shared__ WfThomasLds<double, 2> L;
-    wf_thomas_solve<LC, double, 2>(sp, L, jlo + lane, (int)blockIdx.y, 0);
+    /* a component to a lane also where 16 levels of both (72 spilled
+     * registers) do not fit: 256x256x160, 47.8 us
+     * (51.6 before with 41 of them, 73 in this form of the solve) */
+    constexpr int NC = (LC > 8) ? 1 : 2;
+    __shared__ WfThomasLds<double, NC> L;
+    if constexpr (NC == 1)
+        wf_thomas_solve<LC, double, 1>(sp, L, (int)blockIdx.x * 32 + (lane >> 1), (int)blockIdx.y, lane & 1);
+    else
+        wf_thomas_solve<LC, double, 2>(sp, L, jlo + lane, (int)blockIdx.y, 0);
 #endif
 }
 template <int LC>
@@ -1033,9 +1063,15 @@ hipError_t wf_launch_pivots(const WfSpectral &sp, double *UB, hipStream_t s) {
     return hipGetLastError();
 }
 
+/* workgroups per kx column: 64 systems each, 32 with a component to a lane (see wf_thomas_body) */
+static int wf_thomas_tiles(const WfSpectral &sp) {
+    const int per = (!WF_MIXED && sp.thomas_lc > 8) ? 32 : 64;
+    return (sp.ny + per - 1) / per;
+}
+
 hipError_t wf_launch_thomas(const WfSpectral &sp, hipStream_t s) {
     const int chunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
-    dim3 grd((sp.ny + 63) / 64, sp.hx + sp.low_kx, 1);
+    dim3 grd(wf_thomas_tiles(sp), sp.hx + sp.low_kx, 1);
     if (sp.thomas_lc == 4) {
 #if WF_MIXED
         return hipErrorInvalidValue;
@@ -1114,7 +1150,7 @@ hipError_t wf_launch_fy_batch(const WfSpectral &sp, const WfPressItem *tab, int 
 
 hipError_t wf_launch_thomas_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s) {
     const int chunks = (sp.nz + sp.thomas_lc - 1) / sp.thomas_lc;
-    dim3 grd((sp.ny + 63) / 64, sp.hx + sp.low_kx, nm);
+    dim3 grd(wf_thomas_tiles(sp), sp.hx + sp.low_kx, nm);
     if (sp.thomas_lc == 4) {
 #if WF_MIXED
         return hipErrorInvalidValue;
