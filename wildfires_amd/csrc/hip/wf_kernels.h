@@ -191,7 +191,7 @@ struct WfSpectral {
     double *pmax;        /* npmax partial maxima of |p_new - p_old| (mixed form: then npmax of |p_new|) */
     const wf_real *kx2;  /* hx: kx^2 of the retained x-wavenumbers */
     const wf_real *ky2;  /* ny */
-    const wf_real *ta;   /* nz-1: sub-diagonal a_k (k-only) */
+    const wf_real *ta;   /* nz-1: sub-diagonal a_k (k-only), 0 up to a multiple of 16 */
     const wf_real *tc;   /* nz-1: super-diagonal c_k for k >= 1 (c_0 depends on K^2), 0 up to a multiple of 16 */
     /* the same tables in FP64, for the systems solved in FP64 (all of them in
      * the wf64 compilation, the lowest wavenumbers in the mixed one) */
@@ -204,7 +204,7 @@ struct WfSpectral {
     double dz0, top_div, c0a, c0b; /* c_0 = c0a - 0.5 dz0 K^2 - c0b */
     double b0;                     /* b_0 = -1/dz0 */
     double beta_top;               /* 2/(dz_{Nz-2} dz_{Nz-1}) */
-    const wf_real *beta;           /* nz: 2/(dz_{k-1} dz_k) for 1 <= k <= nz-2 */
+    const wf_real *beta;           /* nz: 2/(dz_{k-1} dz_k) for 1 <= k <= nz-1, 1 up to a multiple of 16 */
     const wf_real *rho;            /* rho^n on every node (variable density) */
     WfIterCtl *ctl;
     WfHostFlag *hflag;             /* mapped host memory */

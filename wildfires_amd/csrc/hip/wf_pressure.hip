@@ -382,8 +382,8 @@ __global__ void k_pivots(WfSpectral sp, double *UB) {
  * of the entry value (products of -L_k, resp. of -c_k/u_k); the waves then
  * combine their chunk ends through LDS in order and add the correction.
  * A lane holds NC components of its system (ky j of kx r): both (64 systems
- * to a wave), or component comp alone (32 systems).  All loads go out first and
- * no level has a branch of its own: the levels above the top read the top's
+ * to a wave), or component comp alone (32 systems).  Loads go out before what
+ * uses them (see SPREAD) and no level has a branch of its own: the levels above the top read the top's
  * entries, and the tables (padded to whole chunks: a = c = 0, beta = 1) keep
  * their values finite and apart from the others. */
 template <typename TA, int NC>
