@@ -9,6 +9,7 @@
 
 #include "wf_common.h"
 #include "wf_closure.h"
+#include "wf_iter.h"
 
 namespace WF_NS {
 
@@ -134,12 +135,12 @@ hipError_t wf_launch_to_reference(const D *src, double *dst, int Nx, int Ny, int
 
 /* Device-side control of the variable-density pressure iteration. */
 struct WfIterCtl {
-    int done;   /* 1 once converged or out of iterations */
+    int done;   /* once converged or out of iterations, 1 + the last solve's index (wf_iter.h) */
     int iters;  /* the count the reference reports */
     int solves; /* solves performed */
     double err; /* last max |p_new - p_old| */
 };
-/* Its copy in mapped host memory, written by every check (done last): the
+/* Its copy in mapped host memory, written by every check (done, 0 or 1, last): the
  * host follows the iteration by it and takes the results from it. */
 struct WfHostFlag {
     int done, solves, iters;

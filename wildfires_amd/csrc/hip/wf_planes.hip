@@ -152,10 +152,10 @@ __device__ __forceinline__ void wf_pl_product(const wf_real *M, int S, const WfP
  * another, so the launch takes enough threads for about two (wf_pl_rhs_nt). */
 template <int MODE>
 __device__ __forceinline__ void wf_pl_rhs_body(const WfConst &c, const WfSpectral &sp, const WfState &Ys,
-                                               const WfState &Yn, const wf_real *p, int block) {
+                                               const WfState &Yn, const wf_real *p, int block, int check) {
     extern __shared__ wf_real smem_r[];
     /* the first solve of a step is never done */
-    const int done = (MODE == WF_F_ITER) ? sp.ctl->done : 0;
+    const int done = (MODE == WF_F_ITER) ? wf_first_pass_returns(sp.ctl->done, check) : 0;
     const int nx = sp.nx, ny = sp.ny, hx = sp.hx, ld = wf_pl_stride(nx + 1);
     const int g = block % sp.pl_groups, ks = block / sp.pl_groups;
     const int k = 1 + ks;
@@ -216,13 +216,13 @@ template <int MODE>
 __global__ __launch_bounds__(512) void k_pl_rhs(WfConst c, WfSpectral sp, WfState Ys, WfState Yn, const wf_real *p,
                                                  double tol, double rtol, int check, int max_iter) {
     const int b = wf_checked_block(sp, tol, rtol, check, max_iter);
-    if (b >= 0) wf_pl_rhs_body<MODE>(c, sp, Ys, Yn, p, b);
+    if (b >= 0) wf_pl_rhs_body<MODE>(c, sp, Ys, Yn, p, b, check);
 }
 template <int MODE>
 __global__ __launch_bounds__(512) void k_pl_rhs_batch(const WfPressItem *__restrict__ tab, int check) {
     const WfPressItem it = wf_press_load(tab);
     const int b = wf_checked_block(it.sp, it.tol, it.rtol, check, it.max_iter);
-    if (b >= 0) wf_pl_rhs_body<MODE>(it.c, it.sp, it.ys, it.yn, it.p, b);
+    if (b >= 0) wf_pl_rhs_body<MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, check);
 }
 
 /* ----------------------------------------------------------------- P2 ---- */
@@ -335,7 +335,7 @@ __device__ __forceinline__ void wf_pl_thomas(const WfSpectral &sp, wf_real *Z, i
 template <int TPW, int LC>
 __device__ __forceinline__ void wf_pl_solve_body(const WfSpectral &sp, int coef) {
     extern __shared__ wf_real smem_r[];
-    const int done = sp.ctl->done;
+    const int done = wf_pass_returns(sp.ctl->done);
     const int ny = sp.ny, nz = sp.nz, hx = sp.hx, hy = wf_pl_half(ny), ld = wf_pl_stride(ny + 1);
     wf_real *Z = smem_r;
     wf_cx<double> *comb = (wf_cx<double> *)(smem_r + (((long)nz * ld + 3) & ~3l));
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(NT) void k_pl_solve_batch(const WfPressItem *__rest
  * (INV = false) or synthesis of WF_PL_LEVELS levels of a plane, in place ... */
 template <bool INV>
 __device__ __forceinline__ void wf_pl_y_body(const WfSpectral &sp) {
-    if (sp.ctl->done) return;
+    if (wf_pass_returns(sp.ctl->done)) return;
     extern __shared__ wf_real smem_r[];
     const int ny = sp.ny, nz = sp.nz, hy = wf_pl_half(ny), ld = wf_pl_stride(ny + 1);
     const int tid = threadIdx.x, nt = (int)blockDim.x;
@@ -546,7 +546,7 @@ __device__ __forceinline__ void wf_pl_y_body(const WfSpectral &sp) {
 /* ... and the tridiagonal solves of 64 systems of a plane, in place. */
 template <int LC>
 __device__ __forceinline__ void wf_pl_tri_body(const WfSpectral &sp) {
-    if (sp.ctl->done) return;
+    if (wf_pass_returns(sp.ctl->done)) return;
     __shared__ wf_cx<double> comb[1024];
     const int coef = blockIdx.x, g = blockIdx.y, nz = sp.nz, hy = wf_pl_half(sp.ny);
     const int r = (coef < sp.hx) ? coef : coef - sp.hx + 1;
@@ -609,7 +609,7 @@ __device__ __forceinline__ void wf_pl_norm(double pv, double pold, double &dmax)
  * (coefficients, old p) goes out before the first wait. */
 __device__ __forceinline__ void wf_pl_inv_body(const WfConst &c, const WfSpectral &sp, wf_real *p) {
     extern __shared__ wf_real smem_r[];
-    const int done = sp.ctl->done;
+    const int done = wf_pass_returns(sp.ctl->done);
     double dmax = 0.0;
     if (blockIdx.x == gridDim.x - 1) {
         if (done) return;

@@ -133,8 +133,8 @@ __global__ __launch_bounds__(WF_NT) void k_iter_check(WfSpectral sp, double tol,
 template <int NX, int MODE>
 __device__ __forceinline__ void wf_rhs_fx_body(const WfConst &c, const WfSpectral &sp, const WfState &Ys,
                                                const WfState &Yn, const wf_real *p, int block, int nblocks,
-                                               const wf_real2 *__restrict__ twx) {
-    if (MODE != WF_F_TOP && sp.ctl->done) return;
+                                               int check, const wf_real2 *__restrict__ twx) {
+    if (MODE != WF_F_TOP && wf_first_pass_returns(sp.ctl->done, check)) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
     constexpr int PAIRS = WfFx<NX>::PAIRS, PER = WfFx<NX>::PER;
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(WF_NT) void k_rhs_fx(WfConst c, WfSpectral sp, WfSt
                                                   const wf_real *p, double tol, double rtol, int check,
                                                   int max_iter, const wf_real2 *__restrict__ twx) {
     const int b = wf_checked_block(sp, tol, rtol, check, max_iter);
-    if (b >= 0) wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p, b, (int)gridDim.x - (check >= 0), twx);
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(c, sp, Ys, Yn, p, b, (int)gridDim.x - (check >= 0), check, twx);
 }
 
 /* P2/P4: y-transform of sp.fy_cols kx columns (each contiguous over ky) of
@@ -279,7 +279,7 @@ __device__ __forceinline__ void wf_fy_f2(const WfSpectral &sp, wf_real2 *base, w
 template <int NY, bool BATCH>
 __device__ __forceinline__ void wf_fy_body(const WfSpectral &sp, wf_real2 *buf, long slab_stride, int slab0, int sign,
                                            int guarded, const wf_real2 *__restrict__ twy) {
-    if (guarded && sp.ctl->done) return;
+    if (guarded && wf_pass_returns(sp.ctl->done)) return;
     extern __shared__ wfc smem[];
     wf_real2 *base = buf + (long)(slab0 + blockIdx.y) * slab_stride;
     const int cols = sp.fy_cols;
@@ -526,7 +526,7 @@ __device__ __forceinline__ void wf_thomas_solve(const WfSpectral &sp, WfThomasLd
 
 template <int LC>
 __device__ __forceinline__ void wf_thomas_body(const WfSpectral &sp) {
-    if (sp.ctl->done) return;
+    if (wf_pass_returns(sp.ctl->done)) return;
     const int lane = threadIdx.x & 63, jlo = blockIdx.x * 64;
 #if WF_MIXED
     /* a tile of 64 systems holding one of the lowest wavenumbers (kx index
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(64 * WF_THOMAS_MAX_CHUNKS) WF_THOMAS_ATTR(LC) void 
  * k_pivots. */
 template <int LC>
 __device__ __forceinline__ void wf_thomas_h_body(const WfSpectral &sp) {
-    if (sp.ctl->done) return;
+    if (wf_pass_returns(sp.ctl->done)) return;
     constexpr int CH = 2 * WF_THOMAS_MAX_CHUNKS;
     __shared__ wf_real2 sv[CH][32];
     __shared__ wf_real sg[CH][32];
@@ -864,7 +864,7 @@ __device__ __forceinline__ void wf_inv_fx_rows(const WfConst &c, const WfSpectra
 template <int NX>
 __device__ __forceinline__ void wf_inv_fx_body(const WfConst &c, const WfSpectral &sp, wf_real *p,
                                                const wf_real2 *__restrict__ twx) {
-    if (sp.ctl->done) return;
+    if (wf_pass_returns(sp.ctl->done)) return;
     extern __shared__ wfc smem[];
     __shared__ int rad[WF_MAX_RADICES];
     if (blockIdx.x == gridDim.x - 1) {
@@ -912,7 +912,7 @@ __global__ __launch_bounds__(WF_NT) void k_rhs_fx_batch(const WfPressItem *__res
                                                         const wf_real2 *__restrict__ twx) {
     const WfPressItem it = wf_press_load(tab);
     const int b = wf_checked_block(it.sp, it.tol, it.rtol, check, it.max_iter);
-    if (b >= 0) wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, (int)gridDim.x - (check >= 0), twx);
+    if (b >= 0) wf_rhs_fx_body<NX, MODE>(it.c, it.sp, it.ys, it.yn, it.p, b, (int)gridDim.x - (check >= 0), check, twx);
 }
 
 /* twy: the class's y twiddle table (it depends on ny alone, so every member's
