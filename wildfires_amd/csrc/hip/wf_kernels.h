@@ -10,6 +10,7 @@
 #include "wf_common.h"
 #include "wf_closure.h"
 #include "wf_iter.h"
+#include "wf_planes_rule.h"
 
 namespace WF_NS {
 
@@ -209,11 +210,11 @@ struct WfSpectral {
     const wf_real *rho;            /* rho^n on every node (variable density) */
     WfIterCtl *ctl;
     WfHostFlag *hflag;             /* mapped host memory */
-    /* coefficient-plane form (wf_planes.hip, FP64), used when pl is set */
+    /* coefficient-plane form (wf_planes.hip, FP64), used when pl is set (wf_pl_takes) */
     int pl;
     int pl_ld;          /* row stride of a plane: ny rounded up to 16 */
     int pl_groups;      /* 16-row groups per slab */
-    int pl_nt;          /* threads of the plane solve; 0: its planes do not fit LDS */
+    int pl_nt;          /* threads of the plane solve; 0: three launches */
     wf_real *U;         /* [nx][nz][pl_ld] planes of real x-coefficients */
     const wf_real *pl_fx, *pl_ix, *pl_fy, *pl_iy; /* MFMA operands of the transforms (wf_pl_matrix) */
     wf_real *pl_l, *pl_ru;  /* [hx][nz up to 16][ny/2+1]: Thomas multipliers l_k and reciprocal pivots 1/u_k */
@@ -238,9 +239,6 @@ hipError_t wf_launch_iter_check(const WfSpectral &sp, double tol, double rtol, i
 
 /* Coefficient-plane form of the solve (wf_planes.hip). */
 #define WF_PL_ROWS 16     /* rows per workgroup in the x-transforms */
-#define WF_PL_LEN_MAX 512 /* longest transform */
-/* whether the form takes an nx x ny x nz solve, and the threads of its plane solve */
-bool wf_pl_takes(int nx, int ny, int nz, int *nt);
 /* MFMA operand tables of a real transform of length n: forward and inverse */
 void wf_pl_matrix(int n, std::vector<double> &fwd, std::vector<double> &inv);
 hipError_t wf_pl_prepare(const WfSpectral &sp, hipStream_t s);

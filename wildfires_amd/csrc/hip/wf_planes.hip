@@ -47,16 +47,8 @@ __device__ __forceinline__ wf_acc wf_mfma(double a, double b, wf_acc c) {
 /* row of accumulator element q in lane group lg = lane / 16 (column lane % 16) */
 __device__ __forceinline__ int wf_acc_row(int lg, int q) { return lg + 4 * q; }
 
-/* LDS row stride of n reals: 4 times an odd number, so that the MFMA operand
- * reads (16 rows x 4 consecutive entries) hit distinct banks */
-__host__ __device__ constexpr int wf_pl_stride(int n) { return 4 * (((n + 3) / 4) | 1); }
 /* levels per workgroup of the transforms of planes that do not fit LDS */
 #define WF_PL_LEVELS 32
-/* levels of the tridiagonal tables: nz rounded up to whole chunks */
-__host__ __device__ constexpr int wf_pl_levels(int nz) { return (nz + 15) & ~15; }
-/* half length (cosine terms) of n, and that rounded up to whole MFMA tiles */
-__host__ __device__ constexpr int wf_pl_half(int n) { return n / 2 + 1; }
-__host__ __device__ constexpr int wf_pl_tiles(int n) { return (wf_pl_half(n) + 15) / 16; }
 
 /* Operand tables of length n, in the order the lanes read them:
  * [tile][step][cos, sin][lane], entry (r, i) = (16 tile + lane % 16,
@@ -464,7 +456,7 @@ __global__ __launch_bounds__(NT) void k_pl_solve_batch(const WfPressItem *__rest
     wf_pl_solve_body<TPW, LC>(it.sp, (int)blockIdx.x);
 }
 
-/* The same in three launches, for planes that do not fit LDS: the y-analysis
+/* The same in three launches (where: wf_pl_solve_nt): the y-analysis
  * (INV = false) or synthesis of WF_PL_LEVELS levels of a plane, in place ... */
 template <bool INV>
 __device__ __forceinline__ void wf_pl_y_body(const WfSpectral &sp) {
@@ -721,52 +713,6 @@ __global__ __launch_bounds__(512) void k_pl_inv_batch(const WfPressItem *__restr
 
 /* ----------------------------------------------------------- launchers ---- */
 
-/* LDS of a plane solve: the plane and the chunk ends of nt threads */
-static size_t wf_pl_lds(int ny, int nz, int nt) {
-    return sizeof(wf_real) * (((size_t)nz * wf_pl_stride(ny + 1) + 3) & ~(size_t)3) + 16 * (size_t)nt;
-}
-#define WF_PL_LDS_MAX (160 * 1024)
-
-/* 16-level tiles per wave and levels per lane of a plane solve of nt threads
- * (0: more than the kernels are built for) */
-static void wf_pl_shape(int ny, int nz, int nt, int *tpw, int *lc) {
-    const int W = nt / 64, T = wf_pl_tiles(ny), nkt = (nz + 15) / 16;
-    const int KG = W / T;
-    const int need = (KG > 0) ? (nkt + KG - 1) / KG : 99;
-    *tpw = (need <= 4) ? need : 0;
-    *lc = ((nz + 3) / 4 * ((ny + 63) / 64) <= W) ? 4 : ((nz + 7) / 8 <= W) ? 8 : ((nz + 15) / 16 <= W) ? 16 : 0;
-}
-
-/* threads of the one-launch plane solve; 0 where the plane does not fit */
-static int wf_pl_solve_nt(int ny, int nz) {
-    for (int n = 256; n <= 1024; n *= 2) {
-        int tpw, lc;
-        wf_pl_shape(ny, nz, n, &tpw, &lc);
-        const int most = (n == 256) ? 1 : (n == 512) ? 2 : 4;
-        if (tpw > 0 && tpw <= most && lc > 0 && lc <= ((n == 1024) ? 16 : 8) && wf_pl_lds(ny, nz, n) <= WF_PL_LDS_MAX)
-            return n;
-    }
-    return 0;
-}
-
-/* lengths with a fast compile-time plan in wf_pressure.hip */
-static bool wf_pl_planned(int n) { return n == 63 || n == 255 || n == 511; }
-
-/* The form takes every solve up to 512 x 512, save those whose lengths both
- * have a compile-time mixed-radix plan and whose y-transforms are long, where
- * n^2/2 multiply-adds cost more than the plan's passes over memory.  us per
- * solve (kernel times, five launches against three):
- *     24x20x16    31 -> 16      100x80x50    91 -> 37     203x60x47  185 -> 41
- *     64x64x32    26 -> 21      128x128x64  102 -> 48     40x200x90  297 -> 110
- *     256x64x64   52 -> 45      256x128x64  137 -> 89     128x256x64 126 -> 95
- *     200x200x90 1553 -> 172    301x301x40  256 -> 232    401x257x40 302 -> 262
- * and, kept on the plans: 64x256x32 38 (49 by planes), 256x256x32 77 (87). */
-bool wf_pl_takes(int nx, int ny, int nz, int *nt) {
-    *nt = wf_pl_solve_nt(ny, nz);
-    if (nx > WF_PL_LEN_MAX || ny > WF_PL_LEN_MAX) return false;
-    return !(wf_pl_planned(nx) && wf_pl_planned(ny) && ny >= 255);
-}
-
 /* threads of P1: enough for two node pairs each, at most 512 (two workgroups
  * a CU, so that one's products run beside the other's loads) */
 static int wf_pl_rhs_nt(const WfSpectral &sp) { return (WF_PL_ROWS * sp.hx <= 512) ? 256 : 512; }
@@ -776,10 +722,6 @@ static int wf_pl_inv_nt(const WfSpectral &sp) {
 }
 static size_t wf_pl_rhs_lds(const WfSpectral &sp) { return sizeof(wf_real) * WF_PL_ROWS * (size_t)wf_pl_stride(sp.nx + 1); }
 static size_t wf_pl_y_lds(const WfSpectral &sp) { return sizeof(wf_real) * WF_PL_LEVELS * (size_t)wf_pl_stride(sp.ny + 1); }
-
-#define WF_PL_SOLVES(X) X(256, 1, 4) X(256, 1, 8) X(512, 1, 4) X(512, 1, 8) X(512, 2, 4) X(512, 2, 8)           \
-    X(1024, 1, 4) X(1024, 1, 8) X(1024, 1, 16) X(1024, 2, 4) X(1024, 2, 8) X(1024, 2, 16) X(1024, 3, 4)         \
-    X(1024, 3, 8) X(1024, 3, 16) X(1024, 4, 4) X(1024, 4, 8) X(1024, 4, 16)
 
 /* tables, and the LDS above 64 KB that the plane solves ask for */
 /* (the x and y passes take at most 133 KB beside their static reductions) */
@@ -835,7 +777,7 @@ hipError_t wf_launch_pl_rhs(const WfConst &c, const WfSpectral &sp, const WfStat
 }
 
 hipError_t wf_launch_pl_solve(const WfSpectral &sp, hipStream_t s) {
-    if (sp.pl_nt == 0) { /* the plane does not fit LDS */
+    if (sp.pl_nt == 0) { /* three launches (wf_pl_solve_nt) */
         const dim3 grd(sp.nx, (sp.nz + WF_PL_LEVELS - 1) / WF_PL_LEVELS), tri(sp.nx, (sp.ny + 63) / 64);
         hipLaunchKernelGGL(k_pl_y<false>, grd, dim3(512), wf_pl_y_lds(sp), s, sp);
         if (sp.nz <= 128)
@@ -847,7 +789,7 @@ hipError_t wf_launch_pl_solve(const WfSpectral &sp, hipStream_t s) {
     }
     int tpw, lc;
     wf_pl_shape(sp.ny, sp.nz, sp.pl_nt, &tpw, &lc);
-    const size_t lds = wf_pl_lds(sp.ny, sp.nz, sp.pl_nt);
+    const size_t lds = (size_t)wf_pl_lds(sp.ny, sp.nz, sp.pl_nt);
 #define WF_PL_GO(NT, TPW, LC)                                                               \
     if (sp.pl_nt == NT && tpw == TPW && lc == LC) {                                         \
         hipLaunchKernelGGL((k_pl_solve<NT, TPW, LC>), dim3(sp.nx), dim3(NT), lds, s, sp);   \
@@ -879,7 +821,7 @@ hipError_t wf_launch_pl_rhs_batch(const WfSpectral &sp, const WfPressItem *tab, 
     return hipGetLastError();
 }
 hipError_t wf_launch_pl_solve_batch(const WfSpectral &sp, const WfPressItem *tab, int nm, hipStream_t s) {
-    if (sp.pl_nt == 0) { /* the plane does not fit LDS */
+    if (sp.pl_nt == 0) { /* three launches (wf_pl_solve_nt) */
         const dim3 grd(sp.nx, (sp.nz + WF_PL_LEVELS - 1) / WF_PL_LEVELS, nm), tri(sp.nx, (sp.ny + 63) / 64, nm);
         hipLaunchKernelGGL(k_pl_y_batch<false>, grd, dim3(512), wf_pl_y_lds(sp), s, tab);
         if (sp.nz <= 128)
@@ -891,7 +833,7 @@ hipError_t wf_launch_pl_solve_batch(const WfSpectral &sp, const WfPressItem *tab
     }
     int tpw, lc;
     wf_pl_shape(sp.ny, sp.nz, sp.pl_nt, &tpw, &lc);
-    const size_t lds = wf_pl_lds(sp.ny, sp.nz, sp.pl_nt);
+    const size_t lds = (size_t)wf_pl_lds(sp.ny, sp.nz, sp.pl_nt);
 #define WF_PL_GO(NT, TPW, LC)                                                                            \
     if (sp.pl_nt == NT && tpw == TPW && lc == LC) {                                                      \
         hipLaunchKernelGGL((k_pl_solve_batch<NT, TPW, LC>), dim3(sp.nx, 1, nm), dim3(NT), lds, s, tab);  \
