@@ -45,3 +45,16 @@ def _against_oracle(tmp_path, nx, ny, nz, form):
 @pytest.mark.parametrize("nx,ny,nz,form", SIZES)
 def test_pressure_form_matches_oracle(tmp_path, nx, ny, nz, form):
     _against_oracle(tmp_path, nx, ny, nz, form)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(64, ny) for ny in range(514, 522)] + [(128, 514), (128, 515), (128, 517), (128, 519)]
+                         + [(256, 515), (256, 517), (256, 519), (256, 521), (512, 514), (512, 515), (512, 516), (512, 517)]
+                         + [(515, 128), (516, 64), (64, 385), (256, 256)])
+def test_fp64_row_maps_match_oracle(tmp_path, nx, ny):
+    """The FP64 x-transforms of the compile-time lengths (their rows of lanes,
+    and the iteration's input by row pairs) on grids that stay on the passes:
+    the last group of 4 (2 at 511) row pairs holding one to all of them, its
+    last pair with a single row or, its second row's upper neighbour being row
+    0, with two; and the compile-time y lengths beside run-time ones in x."""
+    _against_oracle(tmp_path, nx, ny, 6, "passes")
