@@ -7,16 +7,19 @@
  * Ns (natural order, decimation in time): butterfly j in [0, n/R) reads
  * in[j + r n/R], r < R, and writes out[(j/Ns) Ns R + j%Ns + q Ns], q < R, with
  *   out = sum_r W_{Ns R}^{r (j%Ns + q Ns)} in[j + r n/R],  W_m = exp(sign 2 pi i / m).
- * wf_stockham_output states one output element of a stage; it is
- * host/device-neutral, and the CPU check of the plan runs it.
+ * wf_stockham_output states one output element of a stage, for the CPU checks
+ * alone; the kernels run wf_rt_stage, which is host/device-neutral, and a CPU
+ * check compares the two at every length.
  */
 #ifndef WF_FFT_H
 #define WF_FFT_H
 
 #if defined(__HIPCC__)
 #define WF_HD __host__ __device__ __forceinline__
+#define WF_HDM WF_HD
 #else
 #define WF_HD static inline
+#define WF_HDM inline
 #endif
 
 #define WF_MAX_RADICES 16
@@ -86,22 +89,16 @@ WF_HD wfc wf_pack_pair(wfc A, wfc B, int conj) {
     return z;
 }
 
-#if defined(__HIPCC__)
-__device__ __forceinline__ wfc wf_cmul(wfc a, wfc b) {
-#pragma clang fp contract(fast)
-    wfc r;
-    r.re = a.re * b.re - a.im * b.im;
-    r.im = a.re * b.im + a.im * b.re;
-    return r;
-}
-
+#if defined(__cplusplus)
 /* Quotients by a run-time divisor d through its reciprocal rounded up (exact
  * for t < 2^16, d <= 2^10: t (2^32/d + 1) < 2^32 (t/d + 1/d)). */
 struct WfDiv {
     unsigned m;
     int d;
-    __device__ __forceinline__ explicit WfDiv(int div) : m(0xffffffffu / (unsigned)div + 1u), d(div) {}
-    __device__ __forceinline__ int operator()(int t) const { return (d == 1) ? t : (int)__umulhi((unsigned)t, m); }
+    WF_HDM explicit WfDiv(int div) : m(0xffffffffu / (unsigned)div + 1u), d(div) {}
+    WF_HDM int operator()(int t) const {
+        return (d == 1) ? t : (int)(((unsigned long long)(unsigned)t * m) >> 32);
+    }
 };
 
 /* Run-time Stockham stages, wf_stockham_output's terms in its order.  What
@@ -116,10 +113,10 @@ struct WfDiv {
  * length 200 35 -> 24 and 32 -> 21; length 199 (prime) at 200x200x90 y 206 ->
  * 132, x 166 -> 136. */
 template <int R>
-__device__ __forceinline__ void wf_rt_butterfly(const wfc *a, wfc *b, int n, int nseq, int Ns, const wfc *tw) {
+WF_HD void wf_rt_butterfly(const wfc *a, wfc *b, int n, int nseq, int Ns, const wfc *tw, int tid, int nt) {
     const int m = n / R, scale = m / Ns;
     const WfDiv by_m(m), by_ns(Ns);
-    for (int t = threadIdx.x; t < m * nseq; t += blockDim.x) {
+    for (int t = tid; t < m * nseq; t += nt) {
         const int s = by_m(t), j = t - s * m, jq = by_ns(j), kq = j - jq * Ns;
         const wfc *in = a + s * n + j;
         wfc *out = b + s * n + jq * Ns * R + kq;
@@ -144,11 +141,11 @@ __device__ __forceinline__ void wf_rt_butterfly(const wfc *a, wfc *b, int n, int
     }
 }
 #define WF_RT_SEQ 2
-__device__ __forceinline__ void wf_rt_outputs(const wfc *a, wfc *b, int n, int nseq, int R, int Ns, const wfc *tw) {
+WF_HD void wf_rt_outputs(const wfc *a, wfc *b, int n, int nseq, int R, int Ns, const wfc *tw, int tid, int nt) {
     constexpr int S = WF_RT_SEQ;
     const int m = n / R, scale = m / Ns;
     const WfDiv by_n(n), by_ns(Ns), by_r(R);
-    for (int t = threadIdx.x; t < n * (nseq / S); t += blockDim.x) {
+    for (int t = tid; t < n * (nseq / S); t += nt) {
         const int sg = by_n(t), o = t - sg * n;
         const int rest = by_ns(o), kq = o - rest * Ns, jq = by_r(rest), q = rest - jq * R;
         const wfc *in = a + sg * S * n + jq * Ns + kq;
@@ -174,6 +171,21 @@ __device__ __forceinline__ void wf_rt_outputs(const wfc *a, wfc *b, int n, int n
         for (int s = 0; s < S; s++) b[(sg * S + s) * n + o] = acc[s];
     }
 }
+/* Thread tid's part (of nt) of a stage of radix R after radices of product Ns,
+ * over nseq sequences (a multiple of WF_RT_SEQ) of length n, a -> b. */
+WF_HD void wf_rt_stage(const wfc *a, wfc *b, int n, int nseq, int R, int Ns, const wfc *tw, int tid, int nt) {
+    switch (R) {
+        case 2: wf_rt_butterfly<2>(a, b, n, nseq, Ns, tw, tid, nt); break;
+        case 3: wf_rt_butterfly<3>(a, b, n, nseq, Ns, tw, tid, nt); break;
+        case 4: wf_rt_butterfly<4>(a, b, n, nseq, Ns, tw, tid, nt); break;
+        case 5: wf_rt_butterfly<5>(a, b, n, nseq, Ns, tw, tid, nt); break;
+        case 7: wf_rt_butterfly<7>(a, b, n, nseq, Ns, tw, tid, nt); break;
+        default: wf_rt_outputs(a, b, n, nseq, R, Ns, tw, tid, nt); break;
+    }
+}
+#endif
+
+#if defined(__HIPCC__)
 /* One full FFT of `nseq` sequences (a multiple of WF_RT_SEQ) of run-time
  * length n held in LDS (a -> b -> a ...), for lengths without a compile-time
  * plan.  Returns the buffer that holds the result. */
@@ -182,14 +194,7 @@ __device__ __forceinline__ wfc *wf_lds_fft(wfc *a, wfc *b, int n, int nseq, cons
     for (int p = 0; p < WF_MAX_RADICES; p++) {
         const int R = rad[p];
         if (R == 0) break;
-        switch (R) {
-            case 2: wf_rt_butterfly<2>(a, b, n, nseq, Ns, tw); break;
-            case 3: wf_rt_butterfly<3>(a, b, n, nseq, Ns, tw); break;
-            case 4: wf_rt_butterfly<4>(a, b, n, nseq, Ns, tw); break;
-            case 5: wf_rt_butterfly<5>(a, b, n, nseq, Ns, tw); break;
-            case 7: wf_rt_butterfly<7>(a, b, n, nseq, Ns, tw); break;
-            default: wf_rt_outputs(a, b, n, nseq, R, Ns, tw); break;
-        }
+        wf_rt_stage(a, b, n, nseq, R, Ns, tw, (int)threadIdx.x, (int)blockDim.x);
         __syncthreads();
         wfc *tmp = a;
         a = b;
@@ -197,6 +202,14 @@ __device__ __forceinline__ wfc *wf_lds_fft(wfc *a, wfc *b, int n, int nseq, cons
         Ns *= R;
     }
     return a;
+}
+
+__device__ __forceinline__ wfc wf_cmul(wfc a, wfc b) {
+#pragma clang fp contract(fast)
+    wfc r;
+    r.re = a.re * b.re - a.im * b.im;
+    r.im = a.re * b.im + a.im * b.re;
+    return r;
 }
 
 /* ------------------------------------------------------------------------

@@ -357,11 +357,6 @@ __device__ __forceinline__ TA wf_tab(const wf_real *t, const double *td, int i) 
     else
         return (TA)t[i];
 }
-template <typename TA>
-__device__ __forceinline__ wf_cx<TA> wf_ldF(const wf_real2 *F, long i) {
-    const wf_real2 v = F[i];
-    return wf_cx<TA>{(TA)v.x, (TA)v.y};
-}
 
 /* Thomas pivots of every (kx, ky) system (src/cu/pressure.cu:429-433):
  * u_0 = b_0, u_k = b_k - (a_{k-1}/u_{k-1}) c_{k-1}.  They do not change between
