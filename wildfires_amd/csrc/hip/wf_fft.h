@@ -1,9 +1,11 @@
 /*
  * wf_fft.h -- FFT building blocks of the pressure solve.
  *
- * Lengths 63 and 255 (the 64- and 256-node grids) use a two-factor register
- * transform (below).  Any other length runs a mixed-radix Stockham transform
- * in LDS with run-time radices (wf_lds_fft): stage with radix R after radices of product
+ * Lengths 63, 127, 255 and 511 (64 to 512 nodes) have compile-time plans (below):
+ * two factors in registers (y-transforms of 63 and 255), three odd radices with
+ * two of them in registers (FP32 x-transforms of 255), or in place in LDS.  Any
+ * other length runs a mixed-radix Stockham transform in LDS with run-time
+ * radices (wf_lds_fft): stage with radix R after radices of product
  * Ns (natural order, decimation in time): butterfly j in [0, n/R) reads
  * in[j + r n/R], r < R, and writes out[(j/Ns) Ns R + j%Ns + q Ns], q < R, with
  *   out = sum_r W_{Ns R}^{r (j%Ns + q Ns)} in[j + r n/R],  W_m = exp(sign 2 pi i / m).
@@ -557,7 +559,12 @@ __device__ __forceinline__ void wf_f2_phase_b(const wfc *buf, const wf_real2 *tw
  * whose time, bound by them before and by its two phases' latency now, goes
  * from 30.4 to 25.5 us; P1 stays at 32.7 (its loads).  With 4 row pairs to a
  * workgroup instead of 8, 32.6 and 33.2.  In FP64 its registers (145-198)
- * leave too few waves: P5 47 us against 44 in place, P1 84 against 76.
+ * leave too few waves: P5 47 us against 44 in place, P1 84 against 76.  The
+ * form is for three odd radices of which the last is at most PAIRS threads'
+ * share of a workgroup: 255 = 3 5 17 and, of the planned lengths, 63 = 3 3 7,
+ * where it gains nothing (5.2 and 5.4 us in either form, the launch's latency,
+ * at 64x64x32), so it is instantiated for 255 alone; 127 and 511 = 7 73 have
+ * fewer radices.
  * Input of block g of the last radix: x[g + R3 m], m < R1 R2.
  * Phase A: one thread per (sequence, g) runs the radices R1 and R2 on its
  * R1 R2 inputs and twiddles the outputs for the last radix.

@@ -9,27 +9,30 @@
  * y-transformed, solved in z and transformed back by one workgroup in LDS:
  *
  *   P1 k_pl_rhs   : f of 16 rows of a slab, x-analysis      -> planes U[coef][k][j]
- *   P2 k_pl_solve : one plane: y-analysis, Thomas, y-synthesis, in LDS
+ *   P2 k_pl_solve : one plane: y-analysis, Thomas, y-synthesis, in LDS (or, where
+ *                   that does not hold it or measured slower, k_pl_y, k_pl_tri, k_pl_y)
  *   P3 k_pl_inv   : x-synthesis of 16 rows of a slab, p, periodic duplicates,
  *                   max |dp| per workgroup
  *
  * against five dependent launches with the half spectrum read and written
  * three times in between (wf_pressure.hip).  Up to 128 nodes across, a launch
  * of that form takes 4-8 us however little it moves, so the launches were the
- * time; and its run-time radices evaluate a prime factor of the length one
- * output at a time.
+ * time; and its run-time stages evaluate a prime factor p of the length with p
+ * terms to every output.
  *
  * The transforms are products with the cosine and sine matrices on MFMA
  * (v_mfma_f64_16x16x4f64), on the sums and differences
  * x_i +- x_{n-i}, which halve the terms of every output: n^2/2 multiply-adds
  * per real row.  That is the work of a prime length at any factorisation, and
  * costs nothing for the short lengths, where the rows would leave the lanes of
- * a mixed-radix plan idle.
+ * a mixed-radix plan idle; long lengths of small factors stay on the passes
+ * (wf_pl_takes).  Memory: 8 bytes a node for U and 4 for the tables of the
+ * tridiagonal solves (pl_l, pl_ru), where the passes hold 8 and 0.5.
  *
  * FP64 only.  The mixed form's p is a few 1e-5 from the FP64 one, all of it
  * the state's FP32 rounding carried through the divergence, and any other
  * order of operations in its transforms gives another draw of that rounding:
- * as accurate (6e-7 per solve against 6e-7) and 1.3 to 1.7 times as fast when
+ * as accurate (2.6e-7 per solve against 3.7e-7) and 1.3 to 1.7 times as fast when
  * tried, but results that differ by more than its users' comparisons allow.
  */
 #include <math.h>
@@ -110,9 +113,9 @@ struct WfPlMat {
 /* Products of TPW data tiles with one tile of the cosine and sine matrices
  * over S steps (a multiple of 4).  The matrix operands come from L2 (every
  * workgroup reads the same tables), two groups of 4 steps ahead of their use:
- * one group runs for 512 cycles of the matrix core, about what a load takes.  first holds the operands of steps 0 .. 3.  data(s, t,
- * x, y) reads the data operands of step s.  MA: the matrix is the first
- * factor. */
+ * one group runs for 512 cycles of the matrix core, about what a load takes.
+ * first holds the operands of steps 0 .. 3.  data(s, t, x, y) reads the data
+ * operands of step s.  MA: the matrix is the first factor. */
 template <bool MA, int TPW, typename F>
 __device__ __forceinline__ void wf_pl_product(const wf_real *M, int S, const WfPlMat &first, F data,
                                               wf_acc (&c)[TPW], wf_acc (&d)[TPW]) {
@@ -723,8 +726,8 @@ static int wf_pl_inv_nt(const WfSpectral &sp) {
 static size_t wf_pl_rhs_lds(const WfSpectral &sp) { return sizeof(wf_real) * WF_PL_ROWS * (size_t)wf_pl_stride(sp.nx + 1); }
 static size_t wf_pl_y_lds(const WfSpectral &sp) { return sizeof(wf_real) * WF_PL_LEVELS * (size_t)wf_pl_stride(sp.ny + 1); }
 
-/* tables, and the LDS above 64 KB that the plane solves ask for */
-/* (the x and y passes take at most 133 KB beside their static reductions) */
+/* The LDS above 64 KB that the kernels ask for (the x and y passes take at most
+ * 133 KB beside their static reductions). */
 static hipError_t wf_pl_allow(const void *kernel, int bytes = 144 * 1024) {
     return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }

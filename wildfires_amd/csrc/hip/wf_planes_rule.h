@@ -53,7 +53,8 @@ WF_PLR_HD void wf_pl_shape(int ny, int nz, int nt, int *tpw, int *lc) {
  *     16 levels to a lane: 63x63x160 70 | 52, 100x100x160 142 | 101, 256x64x160 165 | 158, 300x10x250 130 | 103
  *     nx <= 128: 64x64x99 57 | 50, 128x128x99 123 | 111, 64x256x64 125 | 93, 128x300x49 164 | 135
  *     above: 144x128x99 128 | 127, 160x64x99 78 | 79, 200x200x63 160 | 168, 401x401x39 476 | 545
- *     one tile to a wave: 127x63x127 55 | 62, 32x280x11 43 | 55, 32x32x99 34 | 31 */
+ *     one tile to a wave: 127x63x127 55 | 62, 32x280x11 43 | 55, 32x32x99 34 | 31
+ * (Three and four tiles to a wave spill 3 and 25 registers.) */
 WF_PLR_HD int wf_pl_solve_nt(int nx, int ny, int nz) {
     for (int n = 256; n <= 1024; n *= 2) {
         int tpw, lc;

@@ -30,14 +30,15 @@
 
 namespace WF_NS {
 
-/* Row pairs of an x-transform workgroup compiled for length NX, and the most
- * elements a thread of it takes.  NX = 0 and -1 are the run-time lengths up
- * to 300 and above. */
 /* FP32 chunks of 8 levels: 8 waves per SIMD, so that two 16-wave workgroups
  * share a CU (256x256x128: 512 workgroups, one round of them) */
 #define WF_THOMAS_ATTR(LC) __attribute__((amdgpu_waves_per_eu((WF_MIXED && (LC) == 8) ? 8 : 4)))
+/* row pairs whose loads are in flight before the one worked on (FP64 P1) */
 #define WF_FX_AHEAD 1
 #define WF_NX_SHORT 300
+/* Row pairs of an x-transform workgroup compiled for length NX, and the most
+ * elements a thread of it takes.  NX = 0 and -1 are the run-time lengths up
+ * to 300 and above. */
 template <int NX>
 struct WfFx {
     static constexpr int LEN = (NX > 0) ? NX : (NX == 0) ? WF_NX_SHORT : 1024;
@@ -532,9 +533,10 @@ __device__ __forceinline__ void wf_thomas_body(const WfSpectral &sp) {
     /* a tile of 64 systems holding one of the lowest wavenumbers (kx index
      * below low_kx, ky index within low_ky of 0 or of ny) is solved in FP64:
      * those systems are singular or nearly so under the Neumann z conditions.
-     * Two workgroups share such a tile, a component of a system to a lane: its
-     * FP64 values then fit the registers of an FP32 workgroup's (64, so that
-     * two of 16 waves share a CU), and its chain of FP64 divisions and
+     * Two workgroups share such a tile, a component of a system to a lane: the
+     * kernel can then be held to 64 registers (two workgroups of 16 waves to a
+     * CU; 18 of the FP64 half's values spill, 68 bytes a lane, which the FP32
+     * tiles do not touch), and its chain of FP64 divisions and
      * combines, the longest of the launch, has half the work.  The second
      * halves are low_kx rows of workgroups before the kx columns'.  us, with
      * a complex FP64 system to a lane, 105 registers and a branch per level

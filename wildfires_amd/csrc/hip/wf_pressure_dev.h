@@ -243,10 +243,11 @@ __device__ __forceinline__ void wf_reduce_max(const double *a, int n, double *ou
  * The check of solve m is done by one extra workgroup (block 0) of solve
  * m + 1's first pass, beside the pass's own workgroups; only the last queued
  * solve is checked by a launch of its own (k_iter_check).  The pass's other
- * workgroups go on whether m converged or not (wf_iter.h).  As its own launch after every solve the check
- * took 4.3-6.2 us of latency, 5 % of a solve at 256x256x128 and 12-17 % at
- * 64x64x32 and below.  (Reducing in the inverse transform itself would need a
- * device-scope release, an L2 write-back, in every workgroup.) */
+ * workgroups go on whether m converged or not (wf_iter.h).  As its own launch
+ * after every solve the check took 4.3-6.2 us of latency, 5 % of a solve at
+ * 256x256x128 and 12-17 % at 64x64x32 and below.  (Reducing in the inverse
+ * transform itself would need a device-scope release, an L2 write-back, in
+ * every workgroup.) */
 __device__ __forceinline__ void wf_iter_check_body(const WfSpectral &sp, double tol, double rtol, int m,
                                                    int max_iter) {
     WfIterCtl *ctl = sp.ctl;
